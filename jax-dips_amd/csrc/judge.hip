@@ -59,52 +59,95 @@ __device__ __forceinline__ float u_entry(const float* __restrict__ u, uint32_t c
   return 0.0f;  // beyond the single ghost layer: cannot occur for stencils of radius 2 around interior points
 }
 
-// y[pt] = (with_c ? c_row : 0) + sum_e w_e u(pt + o_e)   for every record row, one lane per row, entries
-// in order.  Bound by the records' bytes (8 per entry); what held it back was one dependent load chain
-// per entry, so a lane takes kApplyPer entries at a time, all their loads issued before the first use:
-// 95 -> 69 us at 128^3 (15 M entries).  Rows two nodes inside the grid (nearly all) need no ghost
-// test (three below the top of the last axis: codes 125..127, outside the 5^3 cube, decode to 3 there).
+// y[pt] = (with_c ? c_row : 0) + sum_e w_e u(pt + o_e) for every record row, each row's entries in order.
+// Bound by the records' bytes (8 per entry: 118 MB and 25 us at 128^3).  One lane owns a row and adds its
+// entries, but kApplyPer lanes fetch them: a wavefront's load instruction reads 8 rows' next 8 entries (whole
+// lines) instead of one entry of each of 64 rows, all of a round's loads are issued before the first use, and
+// (w, u) reach the owner through LDS.  At 128^3 (star, 15 M entries): 96 us with a lane per row reading its own
+// entries one by one, 57 us with 8 of them in flight, 39 us like this.
+// Workgroups take the rows from the last on, since the records end with their longest rows (33 entries on
+// average next to the interface), which would else start last: 72 against 58 us.  Of each kRowGroup workgroups
+// every die takes neighbours, whose rows read the same u (64 workgroups: 39 us, 128: 40, 512: 58, as one die then
+// has all the long rows).
 // stop (null, or a flag the solver's kernels raise): nothing is done once it is nonzero.
-constexpr int kApplyPer = 8;  // a bulk row's 7 entries in one round
+constexpr int kXcds = 8;
+constexpr int kRowGroup = 64;
+constexpr int kApplyPer = 8;                          // entries of a row per round: a bulk row has 7
+constexpr int kApplyPasses = kApplyPer;               // load instructions per round, 64 / kApplyPer rows each
+constexpr int kPassRows = DIPS_WAVE / kApplyPer;
 __global__ __launch_bounds__(kJudgeThreads) void grid_apply_kernel(
     int nx, int ny, int nz, const int32_t* __restrict__ row_point, const int32_t* __restrict__ row_ptr,
     const float* __restrict__ row_c, int64_t nrows, const uint32_t* __restrict__ ent_code,
     const float* __restrict__ ent_w, int64_t nnz, const float* __restrict__ u, float* __restrict__ y, int with_c,
     const double* __restrict__ stop) {
   if (stop && *stop != 0.0) return;
-  const int64_t row = (int64_t)blockIdx.x * kJudgeThreads + threadIdx.x;
-  if (row >= nrows) return;
-  const int pt = row_point[row];
+  __shared__ int4 rows[kJudgeThreads / DIPS_WAVE][DIPS_WAVE];  // point, first entry, end, whether no ghost is read
+  __shared__ float2 wu[kJudgeThreads / DIPS_WAVE][DIPS_WAVE * (kApplyPer + 1)];  // per row, padded by one
+  const int lane = threadIdx.x & (DIPS_WAVE - 1), wave = threadIdx.x / DIPS_WAVE;
+  const int64_t back = (int64_t)gridDim.x - 1 - blockIdx.x, base = back / kRowGroup * kRowGroup, in = back - base;
+  const int64_t blk =
+      base + kRowGroup <= (int64_t)gridDim.x ? base + (in % kXcds) * (kRowGroup / kXcds) + in / kXcds : back;
+  const int64_t row = blk * kJudgeThreads + threadIdx.x;
   const int64_t npts = (int64_t)nx * ny * nz;
-  if (pt < 0 || pt >= npts) return;
-  const int k = pt % nz, ij = pt / nz, j = ij % ny, i = ij / ny;
-  const int beg = max(row_ptr[row], 0);
-  const int end = (int)min((int64_t)row_ptr[row + 1], nnz);
-  float acc = with_c ? row_c[row] : 0.0f;
-  if (i >= 2 && i < nx - 2 && j >= 2 && j < ny - 2 && k >= 2 && k < nz - 3) {
-    for (int e0 = beg; e0 < end; e0 += kApplyPer) {
-      uint32_t code[kApplyPer];
-      float w[kApplyPer], v[kApplyPer];
+  int pt = -1, beg = 0, end = 0;
+  if (row < nrows) {
+    pt = row_point[row];
+    beg = max(row_ptr[row], 0);
+    end = (int)min((int64_t)row_ptr[row + 1], nnz);
+  }
+  const bool on = pt >= 0 && pt < npts;
+  if (!on) end = beg;
+  {
+    // two nodes inside the grid (three below the top of the last axis: codes 125..127, outside the 5^3 cube,
+    // decode to 3 there)
+    const int k = pt % nz, ij = pt / nz, j = ij % ny, i = ij / ny;
+    const bool inner = on && i >= 2 && i < nx - 2 && j >= 2 && j < ny - 2 && k >= 2 && k < nz - 3;
+    rows[wave][lane] = make_int4(pt, beg, end, inner ? 1 : 0);
+  }
+  float acc = (on && with_c) ? row_c[row] : 0.0f;
+  const int sub = lane % kApplyPer, slot = lane / kApplyPer;
+  __builtin_amdgcn_wave_barrier();
+  for (int c0 = 0; __any(beg + c0 < end); c0 += kApplyPer) {
+    int4 rw[kApplyPasses];
+    uint32_t code[kApplyPasses];
+    float w[kApplyPasses], v[kApplyPasses];
 #pragma unroll
-      for (int q = 0; q < kApplyPer; ++q) {
-        const int e = min(e0 + q, end - 1);
+    for (int q = 0; q < kApplyPasses; ++q) {
+      rw[q] = rows[wave][q * kPassRows + slot];
+      const int e = rw[q].y + c0 + sub;
+      code[q] = 0;
+      w[q] = 0.0f;
+      if (e < rw[q].z) {
         code[q] = ent_code[e];
         w[q] = ent_w[e];
       }
-#pragma unroll
-      for (int q = 0; q < kApplyPer; ++q) {
-        int ox, oy, oz;
-        dips_decode_offset(code[q], ox, oy, oz);
-        v[q] = u[(int64_t)pt + ((int64_t)ox * ny + oy) * nz + oz];
-      }
-#pragma unroll
-      for (int q = 0; q < kApplyPer; ++q)
-        if (e0 + q < end) acc = fmaf(w[q], v[q], acc);
     }
-  } else {
-    for (int e = beg; e < end; ++e) acc = fmaf(ent_w[e], u_entry(u, ent_code[e], i, j, k, nx, ny, nz), acc);
+#pragma unroll
+    for (int q = 0; q < kApplyPasses; ++q) {
+      v[q] = 0.0f;
+      if (rw[q].y + c0 + sub < rw[q].z) {
+        if (rw[q].w) {
+          int ox, oy, oz;
+          dips_decode_offset(code[q], ox, oy, oz);
+          v[q] = u[(int64_t)rw[q].x + ((int64_t)ox * ny + oy) * nz + oz];
+        } else {
+          const int p = rw[q].x, ij = p / nz;
+          v[q] = u_entry(u, code[q], ij / ny, ij % ny, p % nz, nx, ny, nz);
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kApplyPasses; ++q)
+      wu[wave][(q * kPassRows + slot) * (kApplyPer + 1) + sub] = make_float2(w[q], v[q]);
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = 0; q < kApplyPer; ++q) {
+      const float2 p = wu[wave][lane * (kApplyPer + 1) + q];
+      if (beg + c0 + q < end) acc = fmaf(p.x, p.y, acc);
+    }
+    __builtin_amdgcn_wave_barrier();
   }
-  y[pt] = acc;
+  if (on) y[pt] = acc;
 }
 
 // dst = a*x + b*y + c*z (any pointer may alias dst; null operands count as zero)
@@ -195,7 +238,7 @@ __global__ __launch_bounds__(kJudgeThreads) void dot_final_kernel(const double* 
 // The iteration's scalars stay in device memory (the eight doubles behind the partial sums), so that the
 // host waits once per kChunk iterations instead of four times in each, and every vector update also forms the
 // inner products of what it has just computed: 7 launches an iteration, against 20 launches and 4 host waits
-// (at 128^3: 0.50 -> 0.20 ms an iteration, of which the two operator applications take 138 us).
+// (at 128^3: 0.50 -> 0.16 ms an iteration, of which the two operator applications take 78 us).
 // A kernel sums the previous kernel's partial sums itself, in every workgroup.  Once an iteration may not
 // begin (converged, or a breakdown) S[kDone] is raised and the kernels that are still queued do nothing.
 // Slots are written by workgroup 0 only, and never one that another workgroup of the same kernel
