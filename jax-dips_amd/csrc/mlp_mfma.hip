@@ -199,11 +199,21 @@ __device__ __forceinline__ f4 mfma_bf(u4 a, u4 b, f4 c) {
 
 __device__ __forceinline__ float bf_trunc(float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
 
-// bf16 bits of part p of x (the three parts sum to x exactly)
+// bf16 bits of part p of x (the three parts sum to x exactly).  kRound: each part rounded to nearest instead of
+// truncated, |x1| <= 2^-9 |x| and |x2| <= 2^-17 |x| with either sign, which against data split by truncation leaves
+// dropped terms below 2^-23 |a w| without a common sign; costs the packing three conversions instead of masks.
+// There, weights beyond the largest bf16 (infinite ones too) are taken as that: an infinite part times the
+// smaller parts of its data would be NaN, where such a weight saturates its unit; NaN stays NaN.
+template <bool kRound>
 __device__ __forceinline__ uint32_t bf_part(float x, int p) {
-  const float x0 = bf_trunc(x);
+  constexpr float kMax = 3.3895313892515355e38f;
+  if (kRound && fabsf(x) > kMax) x = copysignf(kMax, x);
+  auto part = [](float v) {
+    return kRound ? __uint_as_float((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)v) << 16) : bf_trunc(v);
+  };
+  const float x0 = part(x);
   const float r1 = x - x0;
-  const float x1 = bf_trunc(r1);
+  const float x1 = part(r1);
   const float v = p == 0 ? x0 : (p == 1 ? x1 : r1 - x1);
   return __float_as_uint(v) >> 16;
 }
@@ -219,6 +229,48 @@ __device__ __forceinline__ void bf_split_pair(float x, float y, uint32_t& h, uin
   const float x2 = x1 - __uint_as_float(x1b & 0xffff0000u);
   const float y2 = y1 - __uint_as_float(y1b & 0xffff0000u);
   l = __builtin_amdgcn_perm(__float_as_uint(y2), __float_as_uint(x2), 0x07060302u);
+}
+
+// this lane's units of the three parts of a weight operand (sets `set`, set + 1, set + 2)
+__device__ __forceinline__ void bf_weights(const u4* __restrict__ sets, int set, u4 (&w)[3]) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int p = 0; p < 3; ++p) w[p] = sets[(set + p) * 64 + lane];
+}
+
+// c += the six part products of a weight operand and a data operand (parts h, m, l), smallest terms first
+__device__ __forceinline__ f4 bf6(const u4 (&w)[3], u4 h, u4 m, u4 l, f4 c) {
+  c = mfma_bf(w[2], h, c);
+  c = mfma_bf(w[1], m, c);
+  c = mfma_bf(w[0], l, c);
+  c = mfma_bf(w[1], h, c);
+  c = mfma_bf(w[0], m, c);
+  return mfma_bf(w[0], h, c);
+}
+
+// c[b] += the products of chunk cc: output blocks b = 0 .. NB - 1, weight set set(b, cc).  kAhead: w holds the first
+// block's weights on entry, every operand is read one block ahead of its use, and w holds the next chunk's on
+// return (where there is one); else the compiler places the reads.
+template <int NB, int NC, bool kAhead, class Set>
+__device__ __forceinline__ void bf_chunk(const u4* __restrict__ sets, Set&& set, int cc, u4 h, u4 m, u4 l, u4 (&w)[3],
+                                         f4 (&c)[NB]) {
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    if constexpr (kAhead) {
+      u4 wn[3];
+      const bool more = cc < NC - 1 || b < NB - 1;
+      if (more) bf_weights(sets, b + 1 < NB ? set(b + 1, cc) : set(0, cc + 1), wn);
+      c[b] = bf6(w, h, m, l, c[b]);
+      if (more) {
+#pragma unroll
+        for (int p = 0; p < 3; ++p) w[p] = wn[p];
+      }
+      __builtin_amdgcn_sched_barrier(0);  // keeps the reads in their step
+    } else {
+      bf_weights(sets, set(b, cc), w);
+      c[b] = bf6(w, h, m, l, c[b]);
+    }
+  }
 }
 
 // Packed weights of one phase net for the split-bf16 forward pass:
@@ -240,7 +292,7 @@ struct PackedBf {
   static constexpr int set(int l, int ob, int c, int p) { return (((l - 1) * NB + ob) * NC + c) * 3 + p; }
 };
 
-template <int L, int NB>
+template <int L, int NB, bool kRound = false>
 __device__ void pack_weights_bf(const float* __restrict__ params, FlatNet fn, float* __restrict__ lds) {
   using PK = PackedBf<L, NB>;
   const int Hh = fn.Hh;
@@ -278,14 +330,14 @@ __device__ void pack_weights_bf(const float* __restrict__ params, FlatNet fn, fl
       const int in = 16 * fb + 4 * g + t % 4;
       float w = 0.0f;
       if (fb < NB && in < Hh && out < Hh) w = kTanhExp2Scale * params[fn.w(l) + in * Hh + out];
-      word |= bf_part(w, p) << (16 * h);
+      word |= bf_part<kRound>(w, p) << (16 * h);
     }
     wb[d] = word;
   }
 }
 
 // forward of one tile with the hidden layers on the bf16 matrix cores (layer 0, K = 4, in float32)
-template <int L, int NB>
+template <int L, int NB, bool kAhead = false>
 __device__ __forceinline__ void tile_forward_bf(const float* __restrict__ W, float xin, float (&act)[L][4 * NB]) {
   using PK = PackedBf<L, NB>;
   const int lane = threadIdx.x & 63;
@@ -300,6 +352,8 @@ __device__ __forceinline__ void tile_forward_bf(const float* __restrict__ W, flo
 #pragma unroll
       for (int r = 0; r < 4; ++r) c[ob][r] = W[PK::bias(l) + 16 * ob + 4 * (lane / 16) + r];
     }
+    u4 w[3];
+    if constexpr (kAhead) bf_weights(wb, PK::set(l, 0, 0, 0), w);
 #pragma unroll
     for (int cc = 0; cc < PK::NC; ++cc) {
       u4 ah, am, al;
@@ -314,19 +368,7 @@ __device__ __forceinline__ void tile_forward_bf(const float* __restrict__ W, flo
         am[u] = m;
         al[u] = lo;
       }
-#pragma unroll
-      for (int ob = 0; ob < NB; ++ob) {
-        const u4 w0 = wb[PK::set(l, ob, cc, 0) * 64 + lane];
-        const u4 w1 = wb[PK::set(l, ob, cc, 1) * 64 + lane];
-        const u4 w2 = wb[PK::set(l, ob, cc, 2) * 64 + lane];
-        // smallest terms first
-        c[ob] = mfma_bf(w2, ah, c[ob]);
-        c[ob] = mfma_bf(w1, am, c[ob]);
-        c[ob] = mfma_bf(w0, al, c[ob]);
-        c[ob] = mfma_bf(w1, ah, c[ob]);
-        c[ob] = mfma_bf(w0, am, c[ob]);
-        c[ob] = mfma_bf(w0, ah, c[ob]);
-      }
+      bf_chunk<NB, PK::NC, kAhead>(wb, [&](int ob, int ch) { return PK::set(l, ob, ch, 0); }, cc, ah, am, al, w, c);
     }
 #pragma unroll
     for (int ob = 0; ob < NB; ++ob) {
@@ -667,7 +709,7 @@ struct TransBf {
   static constexpr int set(int l, int ib, int c, int p) { return (((l - 1) * NB + ib) * NC + c) * 3 + p; }
 };
 
-template <int L, int NB>
+template <int L, int NB, bool kRound = false>
 __device__ void pack_trans_bf(const float* __restrict__ params, FlatNet fn, float* __restrict__ lds) {
   using TB = TransBf<L, NB>;
   const int Hh = fn.Hh;
@@ -688,7 +730,7 @@ __device__ void pack_trans_bf(const float* __restrict__ params, FlatNet fn, floa
       const int out = 16 * ob + 4 * g + t % 4;
       float w = 0.0f;
       if (ob < NB && in < Hh && out < Hh) w = kTanhExp2Scale * params[fn.w(l) + in * Hh + out];
-      word |= bf_part(w, p) << (16 * h);
+      word |= bf_part<kRound>(w, p) << (16 * h);
     }
     wb[d] = word;
   }
@@ -854,6 +896,53 @@ __device__ void flush_coop(CoopAcc<L, NB>& G, FlatNet fn, float* __restrict__ re
   for (int i = threadIdx.x; i < P; i += kBT) out[i] = red[i];
 }
 
+// c = W_l d_l of one tile (l >= 1, unscaled by the activation's derivative), d and c feature-major; W is the
+// TransBf copy (kBf: split-bf16 products) or the float32 Packed copy, read transposed
+template <int L, int NB, bool kBf, bool kAhead = false>
+__device__ __forceinline__ void tile_backprop(const float* __restrict__ W, int l, const float (&d)[4 * NB],
+                                              f4 (&c)[NB]) {
+  using PK = Packed<L, NB>;
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int ib = 0; ib < NB; ++ib) c[ib] = f4{0.f, 0.f, 0.f, 0.f};
+  if constexpr (kBf) {
+    // split-bf16: chunk cc of d_l (blocks 2cc, 2cc+1) is the B operand, split like the forward activations
+    using TB = TransBf<L, NB>;
+    const u4* __restrict__ tb = reinterpret_cast<const u4*>(W);
+    u4 w[3];
+    if constexpr (kAhead) bf_weights(tb, TB::set(l, 0, 0, 0), w);
+#pragma unroll
+    for (int cc = 0; cc < TB::NC; ++cc) {
+      u4 dh, dm, dl;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int fb = 2 * cc + u / 2, r = (2 * u) % 4;
+        uint32_t h, mm, lo;
+        bf_split_pair(fb < NB ? d[fb * 4 + r] : 0.0f, fb < NB ? d[fb * 4 + r + 1] : 0.0f, h, mm, lo);
+        dh[u] = h;
+        dm[u] = mm;
+        dl[u] = lo;
+      }
+      bf_chunk<NB, TB::NC, kAhead>(tb, [&](int ib, int ch) { return TB::set(l, ib, ch, 0); }, cc, dh, dm, dl, w, c);
+    }
+  } else {
+    // float32: the A operand of step r over output block fb is W_l[16 ib + m][16 fb + 4 kq + r]
+    // (m = lane%16, kq = lane/16), the float m%4 of unit 16 (m/4) + 4 kq + r of block (fb, ib) -- 4
+    // floats 4 apart from this lane's offset
+    const int m = lane & 15, kq = lane >> 4;
+    const int tofs = 4 * (17 * (m >> 2) + 4 * kq) + (m & 3);
+#pragma unroll
+    for (int fb = 0; fb < NB; ++fb) {
+#pragma unroll
+      for (int ib = 0; ib < NB; ++ib) {
+        const float* wt = W + PK::fwd(l) + (fb * NB + ib) * PK::kBlk + tofs;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) c[ib] = mfma4(wt[4 * r], d[fb * 4 + r], c[ib]);
+      }
+    }
+  }
+}
+
 // kBf: W is the TransBf copy (W_l d_l as split bf16 products), the output weights come in wor and the
 // stage rows are 16 floats with rotated row groups; else W is the float32 Packed copy (float32 MFMA) and
 // the stage rows are padded to kTP floats
@@ -901,53 +990,7 @@ __device__ __forceinline__ void coop_backward(const float* __restrict__ W, const
       // staged copy of d_l), before the barrier: a wavefront that arrives early does this matrix work while
       // it waits.
       f4 c[NB];
-#pragma unroll
-      for (int ib = 0; ib < NB; ++ib) c[ib] = f4{0.f, 0.f, 0.f, 0.f};
-      if constexpr (kBf) {
-        // split-bf16: chunk cc of d_l (blocks 2cc, 2cc+1) is the B operand, split like the forward activations
-        using TB = TransBf<L, NB>;
-        const u4* __restrict__ tb = reinterpret_cast<const u4*>(W);
-#pragma unroll
-        for (int cc = 0; cc < TB::NC; ++cc) {
-          u4 dh, dm, dl;
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int fb = 2 * cc + u / 2, r = (2 * u) % 4;
-            uint32_t h, mm, lo;
-            bf_split_pair(fb < NB ? d[fb * 4 + r] : 0.0f, fb < NB ? d[fb * 4 + r + 1] : 0.0f, h, mm, lo);
-            dh[u] = h;
-            dm[u] = mm;
-            dl[u] = lo;
-          }
-#pragma unroll
-          for (int ib = 0; ib < NB; ++ib) {
-            const u4 w0 = tb[TB::set(l, ib, cc, 0) * 64 + lane];
-            const u4 w1 = tb[TB::set(l, ib, cc, 1) * 64 + lane];
-            const u4 w2 = tb[TB::set(l, ib, cc, 2) * 64 + lane];
-            c[ib] = mfma_bf(w2, dh, c[ib]);
-            c[ib] = mfma_bf(w1, dm, c[ib]);
-            c[ib] = mfma_bf(w0, dl, c[ib]);
-            c[ib] = mfma_bf(w1, dh, c[ib]);
-            c[ib] = mfma_bf(w0, dm, c[ib]);
-            c[ib] = mfma_bf(w0, dh, c[ib]);
-          }
-        }
-      } else {
-        // float32: the A operand of step r over output block fb is W_l[16 ib + m][16 fb + 4 kq + r]
-        // (m = lane%16, kq = lane/16), the float m%4 of unit 16 (m/4) + 4 kq + r of block (fb, ib) -- 4
-        // floats 4 apart from this lane's offset
-        const int m = lane & 15, kq = lane >> 4;
-        const int tofs = 4 * (17 * (m >> 2) + 4 * kq) + (m & 3);
-#pragma unroll
-        for (int fb = 0; fb < NB; ++fb) {
-#pragma unroll
-          for (int ib = 0; ib < NB; ++ib) {
-            const float* wt = W + PK::fwd(l) + (fb * NB + ib) * PK::kBlk + tofs;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) c[ib] = mfma4(wt[4 * r], d[fb * 4 + r], c[ib]);
-          }
-        }
-      }
+      tile_backprop<L, NB, kBf>(W, l, d, c);
 #pragma unroll
       for (int ib = 0; ib < NB; ++ib) {
 #pragma unroll
@@ -1222,139 +1265,133 @@ __global__ void count_inc_kernel(int32_t* count) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *count = *count + 1;
 }
 
-// ---- evaluation at arbitrary points: u and grad_x u (forward mode) ----------------
-// Value and the three input tangents of one 16-position tile, propagated
-// together: a_0 = tanh(W_0 [x,1]), t_0^k = (1 - a_0^2) W_0[k,:]; hidden layers
-// a_l = tanh(W_l a_{l-1} + b_l), t_l^k = (1 - a_l^2) (W_l t_{l-1}^k), sharing each
-// weight operand between the four MFMA chains.  The packed forward weights carry
-// the factor kTanhExp2Scale, which the tangents divide out layer by layer.
-// Returns u and du/dx_k of the tile position lane%16 (identical in the 4 lanes
-// of a position).
-template <int L, int NB>
-__device__ __forceinline__ void tile_value_grad(const float* __restrict__ W, float xin, float& u, float (&du)[3]) {
-  using PK = Packed<L, NB>;
-  const int lane = threadIdx.x & 63;
-  float a[4 * NB], t[3][4 * NB];
-#pragma unroll
-  for (int ob = 0; ob < NB; ++ob) {
-    f4 c = {0.f, 0.f, 0.f, 0.f};
-    c = mfma4(W[PK::l0() + ob * 64 + lane], xin, c);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float v = dips_tanh_exp2(c[r]);
-      const float g = (1.0f - v * v) * (1.0f / kTanhExp2Scale);
-      a[ob * 4 + r] = v;
-#pragma unroll
-      for (int k = 0; k < 3; ++k) t[k][ob * 4 + r] = g * W[PK::l0() + ob * 64 + 16 * k + 4 * (lane / 16) + r];
+// ---- evaluation at arbitrary points: u and grad_x u --------------------------------
+// The training step's tile passes: the forward pass in FwdPack's copy and, for grad u, one
+// back-propagation of d u / d u = 1 down to the inputs (kGrad) in the backward's copy; u alone otherwise.  Bound by
+// the matrix and VALU work of those two passes.  3x64 at 256^3 points with grad u: 3.7 ms; value and three input
+// tangents propagated forward together in float32 MFMA: 10.4 ms (four chains of products instead
+// of two, each 2.7x the matrix cycles of the split-bf16 ones).
+// A workgroup packs the + network, takes its tiles of 16 consecutive points that hold a + point, then the same for
+// the - network: both networks' copies do not fit in LDS beside each other, and this way every workgroup has
+// the same mix of the two whatever the share of the phases.
+template <int L, int NB, bool kGrad>
+struct EvalPhase {
+  static constexpr bool kBf = FwdPack<L, NB>::kBf;
+  static constexpr int fwd() { return (FwdPack<L, NB>::size() + 3) & ~3; }
+  static constexpr int floats() { return fwd() + (kGrad && kBf ? TransBf<L, NB>::size() : 0); }
+};
+template <int Lm, int NBm, int Lp, int NBp, bool kGrad>
+struct EvalCfg {
+  static constexpr int kP = EvalPhase<Lp, NBp, kGrad>::floats(), kM = EvalPhase<Lm, NBm, kGrad>::floats();
+  static constexpr int kFloats = kP > kM ? kP : kM;
+  // Where the copies take more than half of the LDS (3x64 with grad u, 100 KB) one workgroup of 12 wavefronts with
+  // 168 registers each (256^3 points: 3.70 ms; 16 of 128, which spill: 4.85; 8 of 256: 4.16), else
+  // workgroups of 8, six wavefronts per SIMD for u alone (1.75 ms; four: 1.94).
+  static constexpr bool kWide = kFloats * sizeof(float) > 80 * 1024;
+  static constexpr int kThreads = kWide ? 768 : 512;
+  static constexpr int kWavesPerSimd = kWide ? 3 : kGrad ? 4 : 6;
+};
+
+struct EvalArgs {
+  const float* pts;
+  const uint8_t* phase;
+  const float* nrm;
+  int64_t m;
+  float* u;
+  float* grad;
+  float* gradn;
+};
+
+// the tiles of this workgroup that hold a point of phase kPlus
+template <int L, int NB, bool kGrad, bool kPlus>
+__device__ __forceinline__ void eval_phase(const EvalArgs& E, const float* __restrict__ params, FlatNet fn,
+                                           float* __restrict__ lds) {
+  using EP = EvalPhase<L, NB, kGrad>;
+  using PK = std::conditional_t<EP::kBf, PackedBf<L, NB>, Packed<L, NB>>;
+  const float* const bwdW = EP::kBf ? lds + EP::fwd() : lds;  // the float32 copy serves both passes
+  if constexpr (EP::kBf)
+    pack_weights_bf<L, NB, true>(params, fn, lds);
+  else
+    pack_weights<L, NB>(params, fn, lds);
+  if constexpr (kGrad && EP::kBf) pack_trans_bf<L, NB, true>(params, fn, lds + EP::fwd());
+  __syncthreads();
+  const int lane = threadIdx.x & 63, k = lane / 16;
+  const int64_t waves = blockDim.x / 64, ntiles = (E.m + 15) / 16, step = (int64_t)gridDim.x * waves;
+  int64_t tile = (int64_t)blockIdx.x * waves + threadIdx.x / 64;
+  // a tile's points and phases are loaded one tile ahead
+  auto load = [&](int64_t t, float& x, bool& mine) {
+    const int64_t p = t * 16 + (lane & 15);
+    x = k == 3 ? 1.0f : 0.0f;
+    mine = false;
+    if (p < E.m) {
+      if (k < 3) x = E.pts[3 * p + k];
+      mine = (E.phase[p] != 0) == kPlus;
     }
-  }
+  };
+  float x_next;
+  bool mine_next;
+  load(tile, x_next, mine_next);
+  for (; tile < ntiles; tile += step) {
+    const float xin = x_next;
+    const bool mine = mine_next;
+    load(tile + step, x_next, mine_next);
+    if (!__any(mine)) continue;
+    const int64_t p = tile * 16 + (lane & 15);
+    float act[L][4 * NB];
+    if constexpr (EP::kBf)
+      tile_forward_bf<L, NB, true>(lds, xin, act);
+    else
+      tile_forward<L, NB>(lds, xin, act);
+    const float u = tile_output<L, NB, PK>(lds, act);
+    if constexpr (kGrad) {
+      float d[4 * NB];
 #pragma unroll
-  for (int l = 1; l < L; ++l) {
-    f4 c[NB], ct[3][NB];
+      for (int q = 0; q < 4 * NB; ++q) {
+        const float a = act[L - 1][q];
+        d[q] = lds[PK::wout() + 16 * (q / 4) + 4 * k + q % 4] * (1.0f - a * a);
+      }
 #pragma unroll
-    for (int ob = 0; ob < NB; ++ob) {
+      for (int l = L - 1; l >= 1; --l) {
+        f4 c[NB];
+        tile_backprop<L, NB, EP::kBf, true>(bwdW, l, d, c);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) c[ob][r] = W[PK::bias(l) + 16 * ob + 4 * (lane / 16) + r];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) ct[k][ob] = f4{0.f, 0.f, 0.f, 0.f};
-    }
-#pragma unroll
-    for (int fb = 0; fb < NB; ++fb) {
-#pragma unroll
-      for (int ob = 0; ob < NB; ++ob) {
-        const f4 w4 = *reinterpret_cast<const f4*>(&W[PK::fwd(l) + (ob * NB + fb) * PK::kBlk + 4 * PK::unit(lane)]);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          c[ob] = mfma4(w4[r], a[fb * 4 + r], c[ob]);
-#pragma unroll
-          for (int k = 0; k < 3; ++k) ct[k][ob] = mfma4(w4[r], t[k][fb * 4 + r], ct[k][ob]);
+        for (int q = 0; q < 4 * NB; ++q) {
+          const float a = act[l - 1][q];
+          d[q] = c[q / 4][q % 4] * (1.0f - a * a);
         }
       }
-    }
+      // d u / d x_i = sum_j W_0[i][j] d_j; every packed layer carries the factor kTanhExp2Scale
+      float scale = 1.0f;
 #pragma unroll
-    for (int ob = 0; ob < NB; ++ob) {
+      for (int l = 0; l < L; ++l) scale *= 1.0f / kTanhExp2Scale;
+      float g[3];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float v = dips_tanh_exp2(c[ob][r]);
-        const float g = (1.0f - v * v) * (1.0f / kTanhExp2Scale);
-        a[ob * 4 + r] = v;
+      for (int i = 0; i < 3; ++i) {
+        float t = 0.0f;
 #pragma unroll
-        for (int k = 0; k < 3; ++k) t[k][ob * 4 + r] = g * ct[k][ob][r];
+        for (int q = 0; q < 4 * NB; ++q) t = fmaf(lds[PK::l0() + (q / 4) * 64 + 16 * i + 4 * k + q % 4], d[q], t);
+        t += __shfl_xor(t, 16, 64);
+        t += __shfl_xor(t, 32, 64);
+        g[i] = t * scale;
+      }
+      if (mine) {
+        if (k < 3 && E.grad) E.grad[3 * p + k] = k == 0 ? g[0] : k == 1 ? g[1] : g[2];
+        if (k == 3 && E.gradn) E.gradn[p] = g[0] * E.nrm[3 * p] + g[1] * E.nrm[3 * p + 1] + g[2] * E.nrm[3 * p + 2];
       }
     }
+    if (mine && k == 0) E.u[p] = u;
   }
-  float s = 0.0f, d0 = 0.0f, d1 = 0.0f, d2 = 0.0f;
-#pragma unroll
-  for (int fb = 0; fb < NB; ++fb) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float wo = W[PK::wout() + 16 * fb + 4 * (lane / 16) + r];
-      s = fmaf(a[fb * 4 + r], wo, s);
-      d0 = fmaf(t[0][fb * 4 + r], wo, d0);
-      d1 = fmaf(t[1][fb * 4 + r], wo, d1);
-      d2 = fmaf(t[2][fb * 4 + r], wo, d2);
-    }
-  }
-  s += __shfl_xor(s, 16, 64);
-  s += __shfl_xor(s, 32, 64);
-  d0 += __shfl_xor(d0, 16, 64);
-  d0 += __shfl_xor(d0, 32, 64);
-  d1 += __shfl_xor(d1, 16, 64);
-  d1 += __shfl_xor(d1, 32, 64);
-  d2 += __shfl_xor(d2, 16, 64);
-  d2 += __shfl_xor(d2, 32, 64);
-  u = s + W[PK::bout()];
-  du[0] = d0;
-  du[1] = d1;
-  du[2] = d2;
 }
 
-// u, grad u and grad u . n at m points; both networks packed once per
-// workgroup (+ net first); a wavefront takes 16 consecutive points and runs
-// each network only if one of its points selects it.
-template <int Lm, int NBm, int Lp, int NBp>
-__global__ __launch_bounds__(kMT) void mfma_eval_kernel(const float* __restrict__ params, int Hm, int Hp,
-                                                        const float* __restrict__ pts,
-                                                        const uint8_t* __restrict__ phase,
-                                                        const float* __restrict__ nrm, int64_t m,
-                                                        float* __restrict__ u, float* __restrict__ grad,
-                                                        float* __restrict__ gradn) {
+template <int Lm, int NBm, int Lp, int NBp, bool kGrad>
+__global__ __launch_bounds__((EvalCfg<Lm, NBm, Lp, NBp, kGrad>::kThreads),
+                             (EvalCfg<Lm, NBm, Lp, NBp, kGrad>::kWavesPerSimd)) void
+mfma_eval_kernel(const float* __restrict__ params, int Hm, int Hp, EvalArgs E) {
   extern __shared__ __align__(16) float lds[];
-  constexpr int kOffM = (Packed<Lp, NBp>::size() + 3) & ~3;  // the - net starts 16-byte aligned
-  const int wave = threadIdx.x / 64, lane = threadIdx.x & 63;
   const int PPp = 4 * Hp + (Lp - 1) * (Hp * Hp + Hp) + Hp + 1;
-  pack_weights<Lp, NBp>(params, FlatNet{Hp, Lp, 0}, lds);
-  pack_weights<Lm, NBm>(params, FlatNet{Hm, Lm, PPp}, lds + kOffM);
+  eval_phase<Lp, NBp, kGrad, true>(E, params, FlatNet{Hp, Lp, 0}, lds);
   __syncthreads();
-  const int64_t ntiles = (m + 15) / 16;
-  for (int64_t tile = (int64_t)blockIdx.x * 4 + wave; tile < ntiles; tile += (int64_t)gridDim.x * 4) {
-    const int64_t p = tile * 16 + (lane & 15);
-    const bool valid = p < m;
-    float x = 0.0f, y = 0.0f, z = 0.0f;
-    bool plus = false;
-    if (valid) {
-      x = pts[3 * p];
-      y = pts[3 * p + 1];
-      z = pts[3 * p + 2];
-      plus = phase[p] != 0;
-    }
-    const int k = lane / 16;
-    const float xin = (k == 0) ? x : (k == 1) ? y : (k == 2) ? z : 1.0f;
-    float up = 0.0f, um = 0.0f, gp[3] = {0.f, 0.f, 0.f}, gm[3] = {0.f, 0.f, 0.f};
-    if (__any(valid && plus)) tile_value_grad<Lp, NBp>(lds, xin, up, gp);
-    if (__any(valid && !plus)) tile_value_grad<Lm, NBm>(lds + kOffM, xin, um, gm);
-    if (valid && lane < 16) {
-      const float v = plus ? up : um;
-      const float g0 = plus ? gp[0] : gm[0], g1 = plus ? gp[1] : gm[1], g2 = plus ? gp[2] : gm[2];
-      u[p] = v;
-      if (grad) {
-        grad[3 * p] = g0;
-        grad[3 * p + 1] = g1;
-        grad[3 * p + 2] = g2;
-      }
-      if (gradn && nrm) gradn[p] = g0 * nrm[3 * p] + g1 * nrm[3 * p + 1] + g2 * nrm[3 * p + 2];
-    }
-  }
+  eval_phase<Lm, NBm, kGrad, false>(E, params, FlatNet{Hm, Lm, PPp}, lds);
 }
 
 // loss = inv_b * sum of the row-sum partials (fixed order), gradient copy-out
@@ -1437,33 +1474,6 @@ int64_t mfma_workspace_floats(const dips_net_t* n, int64_t max_rows, int64_t max
   return mfma_base_floats(n, max_rows, max_nnz) + 64 + (max_nnz / 16 + 2) * (int64_t)act_f4_of(n) * 256;
 }
 
-// dips_eval for the network shapes of the MFMA path
-int mfma_eval_launch(const dips_net_t* net, const float* params, const float* pts, const uint8_t* phase,
-                     const float* nrm, int64_t m, float* u, float* grad, float* gradn, hipStream_t st) {
-  if (!mfma_supported(net)) {
-    set_error("dips_eval: network shape has no compiled kernel");
-    return DIPS_EUNSUPPORTED;
-  }
-  if (m <= 0) return DIPS_OK;
-  const int Hm = net->Hm, Hp = net->Hp;
-  const int a = net->Lm, b = nb_of(Hm), c = net->Lp, d = nb_of(Hp);
-  const int64_t ntiles = (m + 15) / 16;
-  const int nblk = (int)std::min<int64_t>((ntiles + 3) / 4, 1024);
-#define X(A, B, C, D)                                                                                            \
-  if (a == A && b == B && c == C && d == D) {                                                                   \
-    const size_t lds = sizeof(float) * (((Packed<C, D>::size() + 3) & ~3) + Packed<A, B>::size());             \
-    hipFuncSetAttribute((const void*)mfma_eval_kernel<A, B, C, D>, hipFuncAttributeMaxDynamicSharedMemorySize,  \
-                        (int)lds);                                                                             \
-    hipLaunchKernelGGL((mfma_eval_kernel<A, B, C, D>), dim3(nblk), dim3(kMT), lds, st, params, Hm, Hp, pts, phase, \
-                       nrm, m, u, grad, gradn);                                                                 \
-    return hip_status(hipGetLastError(), "mfma_eval_kernel launch");                                            \
-  }
-  DIPS_MFMA_SHAPES(X)
-#undef X
-  set_error("dips_eval: network shape has no compiled kernel");
-  return DIPS_EUNSUPPORTED;
-}
-
 // Workgroups of a persistent kernel resident at once on the current device
 // (compute units x occupancy), looked up once per kernel and device; fallback
 // if the runtime cannot say.  A persistent grid of exactly this size runs in
@@ -1483,6 +1493,48 @@ int resident_blocks(const void* fn, int threads, size_t lds, int fallback) {
     n = per_cu * cus;
   cache.push_back({{fn, dev}, n});
   return n;
+}
+
+// dips_eval for the network shapes of the MFMA path
+int mfma_eval_launch(const dips_net_t* net, const float* params, const float* pts, const uint8_t* phase,
+                     const float* nrm, int64_t m, float* u, float* grad, float* gradn, hipStream_t st) {
+  if (!mfma_supported(net)) {
+    set_error("dips_eval: network shape has no compiled kernel");
+    return DIPS_EUNSUPPORTED;
+  }
+  if (m <= 0) return DIPS_OK;
+  const int Hm = net->Hm, Hp = net->Hp;
+  const int a = net->Lm, b = nb_of(Hm), c = net->Lp, d = nb_of(Hp);
+  const int64_t ntiles = (m + 15) / 16;
+  const EvalArgs E{pts, phase, nrm, m, u, grad, nrm ? gradn : nullptr};
+#define Y(A, B, C, D, G)                                                                                         \
+  {                                                                                                              \
+    using Cfg = EvalCfg<A, B, C, D, G>;                                                                          \
+    constexpr size_t lds = sizeof(float) * Cfg::kFloats;                                                         \
+    static const bool attr_set = hipFuncSetAttribute((const void*)mfma_eval_kernel<A, B, C, D, G>,               \
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) ==    \
+                                 hipSuccess;                                                                     \
+    (void)attr_set;                                                                                              \
+    const int64_t waves = Cfg::kThreads / 64;                                                                    \
+    const int nblk = (int)std::min<int64_t>((ntiles + waves - 1) / waves,                                        \
+                                            resident_blocks((const void*)mfma_eval_kernel<A, B, C, D, G>,        \
+                                                            Cfg::kThreads, lds, 256));                           \
+    hipLaunchKernelGGL((mfma_eval_kernel<A, B, C, D, G>), dim3(nblk), dim3(Cfg::kThreads), lds, st, params, Hm,  \
+                       Hp, E);                                                                                   \
+    return hip_status(hipGetLastError(), "mfma_eval_kernel launch");                                             \
+  }
+#define X(A, B, C, D)                         \
+  if (a == A && b == B && c == C && d == D) { \
+    if (grad || E.gradn)                      \
+      Y(A, B, C, D, true)                     \
+    else                                      \
+      Y(A, B, C, D, false)                    \
+  }
+  DIPS_MFMA_SHAPES(X)
+#undef X
+#undef Y
+  set_error("dips_eval: network shape has no compiled kernel");
+  return DIPS_EUNSUPPORTED;
 }
 
 // opt == nullptr: stop after the reduction (gradient in grad_out, loss in loss_out)
