@@ -10,8 +10,9 @@
 // layer, so layers chain without data movement.  Weight operands are packed
 // once per workgroup into LDS in that order.  Weight gradients contract over
 // positions, so the two operands (activation and delta of a tile) pass through
-// a padded LDS transpose and the 16x16 dW blocks accumulate in AGPRs across
-// all tiles of the wavefront.
+// an LDS transpose (bf16 parts and transposing reads for 64-wide networks,
+// float32 rows for narrower ones) and the dW blocks accumulate in registers
+// across all rounds of a group of wavefronts.
 //
 // Per optimizer step: fwd (u per entry) -> rowsum (r per row, loss partials)
 // -> bwd (parameter-gradient partials per workgroup) -> reduce -> apply.
@@ -37,7 +38,7 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 
 constexpr int kMT = 256;  // threads per workgroup (4 wavefronts)
 constexpr int kTP = 20;   // padded row length of a transposed 16-position tile (16-byte aligned rows)
-constexpr int kMfmaBwdBlocks = 512;   // workgroups of the backward kernel (both phases), two per CU
+constexpr int kMfmaBwdGroups = 512;   // groups of 4 wavefronts of the backward kernel (both phases), two per CU
 constexpr int kMfmaFwdBlocks = 1024;  // workgroups of the forward kernel (both phases), four per CU
 
 __device__ __forceinline__ f4 mfma4(float a, float b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
@@ -129,18 +130,6 @@ __device__ __forceinline__ void tile_layer0(const float* __restrict__ W, float x
   }
 }
 
-// layer 0 from this lane's operands held in registers (w0[ob] = the packed value at ob * 64 + lane)
-template <int L, int NB>
-__device__ __forceinline__ void tile_layer0_regs(const float (&w0)[NB], float xin, float (&act)[L][4 * NB]) {
-#pragma unroll
-  for (int ob = 0; ob < NB; ++ob) {
-    f4 c = {0.f, 0.f, 0.f, 0.f};
-    c = mfma4(w0[ob], xin, c);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) act[0][ob * 4 + r] = dips_tanh_exp2(c[r]);
-  }
-}
-
 // forward of one tile: act[l][fb*4+r] feature-major; returns nothing (u by caller)
 template <int L, int NB>
 __device__ __forceinline__ void tile_forward(const float* __restrict__ W, float xin, float (&act)[L][4 * NB]) {
@@ -192,6 +181,7 @@ __device__ __forceinline__ void tile_forward(const float* __restrict__ W, float 
 // of blocks 2c and 2c+1, split, and layers still chain without data movement.
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ f4 mfma_bf(u4 a, u4 b, f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, a), __builtin_bit_cast(bf8, b), c, 0, 0, 0);
@@ -679,21 +669,20 @@ __global__ __launch_bounds__(256) void mfma_seed_kernel(MfmaTileArgs T, int64_t 
 }
 
 // ---- kernel 3: parameter-gradient partials ---------------------------------------
-// Cooperative backward: a workgroup of kBW wavefronts takes kBW tiles of one
-// phase per round.  Every wavefront recomputes its tile's forward pass and
-// back-propagates its deltas (registers); per layer, each wavefront stages its
-// tile's operands (activation and delta, feature-major rows of 16 positions)
-// in LDS, and after a barrier each wavefront contracts only the weight-gradient
-// blocks it owns over all kBW tiles (K = 16 kBW positions).  Owning 4 of the
-// 16 blocks of a 64-wide layer keeps a lane's registers within 256, and the
-// packed weights (one copy, read transposed for the deltas) plus the stage fit
-// twice into a CU's LDS: two workgroups per CU, whose barriers are independent,
-// so one workgroup's wavefronts issue while the other's wait.
-// Bias, output-weight and output-bias sums stay per lane and are reduced over
+// Cooperative backward: a group of kBW wavefronts takes kBW tiles of one
+// phase per round.  Every wavefront back-propagates its tile's deltas
+// (registers); per layer, each wavefront stages its tile's operands
+// (activation and delta) in LDS, and after a barrier each wavefront contracts
+// only the weight-gradient blocks it owns over all kBW tiles (K = 16 kBW
+// positions).  Owning a quarter of a 64-wide layer keeps a lane's registers
+// within 256: two wavefronts per SIMD, of two groups that overlap (two
+// workgroups with barriers of their own, or two groups of one workgroup a
+// barrier apart, see bwd_groups), so that one group issues while the other waits.
+// Output-weight and output-bias sums stay per lane and are reduced over
 // the 16 positions with row-local DPP sums at the end.  The packed weights carry
 // the factor kTanhExp2Scale, so each layer's delta comes out that factor larger
 // than the one after it; the flush divides it out.
-constexpr int kBW = 4;              // wavefronts per backward workgroup
+constexpr int kBW = 4;              // wavefronts per backward group
 constexpr int kBT = 64 * kBW;       // its threads
 
 // Transposed split-bf16 copy of the hidden matrices for the backward pass: per hidden
@@ -736,26 +725,92 @@ __device__ void pack_trans_bf(const float* __restrict__ params, FlatNet fn, floa
   }
 }
 
-// this lane's layer-0 operands (the packed value at ob * 64 + lane) and output weights (feature
-// 16 fb + 4 (lane / 16) + r at fb * 4 + r), for the backward pass without the float32 copy in LDS
+// layer 0's operands (the packed value at ob * 64 + lane) and the output weights of the backward pass with TransBf
 template <int NB>
-__device__ __forceinline__ void lane_weights(const float* __restrict__ params, FlatNet fn, float (&w0)[NB],
-                                             float (&wo)[4 * NB]) {
-  const int lane = threadIdx.x & 63, Hh = fn.Hh;
-#pragma unroll
-  for (int ob = 0; ob < NB; ++ob) {
-    const int out = 16 * ob + lane % 16, k = lane / 16;
-    w0[ob] = out < Hh ? kTanhExp2Scale * ((k < 3) ? params[fn.w(0) + k * Hh + out] : params[fn.b(0) + out]) : 0.0f;
-  }
-#pragma unroll
-  for (int q = 0; q < 4 * NB; ++q) {
-    const int h = 16 * (q / 4) + 4 * (lane / 16) + q % 4;
-    wo[q] = h < Hh ? params[fn.wout() + h] : 0.0f;
+__device__ void pack_edges(const float* __restrict__ params, FlatNet fn, float* __restrict__ lds) {
+  const int Hh = fn.Hh;
+  for (int idx = threadIdx.x; idx < 80 * NB; idx += blockDim.x) {
+    float v = 0.0f;
+    if (idx < NB * 64) {
+      const int out = 16 * (idx / 64) + idx % 16, k = idx % 64 / 16;
+      if (out < Hh) v = kTanhExp2Scale * ((k < 3) ? params[fn.w(0) + k * Hh + out] : params[fn.b(0) + out]);
+    } else if (idx - NB * 64 < Hh) {
+      v = params[fn.wout() + idx - NB * 64];
+    }
+    lds[idx] = v;
   }
 }
 
+// 64-wide networks (NB = 4): the weight gradients as split-bf16 products as well (SplitAcc, split_backward).
+// A K = 16 product over one tile's positions needs, per lane, 8 positions of one feature, while a tile's registers
+// hold 4 features of one position: every wavefront stages its activations' and deltas' parts as 8-byte units (bf16
+// features 4 g .. 4 g + 3 of block fb at position p, the registers of lane 16 g + p), and ds_read_b64_tr_b16 hands
+// 4 positions of a feature to each lane.  Unit (fb, g, p) lies at place p ^ 4 (g / 2) of the 16 of (fb, g): a
+// wavefront writes 512 consecutive bytes, and the 64 units of a transposing read (2 fb, 4 g, positions a .. a + 3
+// and a + 8 .. a + 11) fill each bank twice, the least there is.  Measured per wavefront instruction: write 6.3 and read 2.2
+// cycles; rows of positions padded to 72 halves: 8.1 and 4.0.
+template <int NB>
+struct SplitStage {
+  static constexpr int kPart = 16 * 16 * NB;    // halves of one part of a tile's operand
+  static constexpr int kOperand = 3 * kPart;
+  static constexpr int kTile = 2 * kOperand;    // activations, then deltas
+  static constexpr int kInPart = 16 * 4;        // layer 0: the inputs' parts, [position][4], at the activations' place
+  static constexpr int floats() { return kTile / 2; }
+  static __device__ __forceinline__ int unit(int fb, int g, int p) { return 256 * fb + 64 * g + 4 * (p ^ (4 * (g >> 1))); }
+};
+typedef float f16v __attribute__((ext_vector_type(16)));
+typedef short s4v __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f16v mfma_bf32(u4 a, u4 b, f16v c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8, a), __builtin_bit_cast(bf8, b), c, 0, 0, 0);
+}
+// two transposing reads: of the 16 lanes of a group, lane i gives the address of position i / 4's 4 features
+// 4 (i % 4) .. at `lo` (and of position 4 + i / 4 at `hi`) and receives feature i's 4 + 4 positions
+__device__ __forceinline__ u4 tr_read8(const uint16_t* lo, const uint16_t* hi) {
+  typedef __attribute__((address_space(3))) s4v lds_s4v;
+  struct {
+    s4v a, b;
+  } v{__builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4v*)lo), __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4v*)hi)};
+  return __builtin_bit_cast(u4, v);
+}
+// stages the parts of chunk cc (blocks 2cc, 2cc + 1) of a feature-major tile matrix
+template <int NB>
+__device__ __forceinline__ void split_stage(uint16_t* operand, int cc, u4 h, u4 m, u4 l) {
+  using SS = SplitStage<NB>;
+  typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+  const int lane = threadIdx.x & 63;
+  uint16_t* at = operand + SS::unit(2 * cc, lane >> 4, lane & 15);
+#pragma unroll
+  for (int f = 0; f < 2; ++f) {
+    *reinterpret_cast<u2*>(at + 256 * f) = u2{h[2 * f], h[2 * f + 1]};
+    *reinterpret_cast<u2*>(at + SS::kPart + 256 * f) = u2{m[2 * f], m[2 * f + 1]};
+    *reinterpret_cast<u2*>(at + 2 * SS::kPart + 256 * f) = u2{l[2 * f], l[2 * f + 1]};
+  }
+}
+template <int L, int NB>
+struct SplitAcc {
+  static constexpr bool kSplit = true;
+  f16v dW[L > 1 ? L - 1 : 1];           // hidden-layer 32x32 block (wave / 2, wave % 2)
+  f4 dW0;                               // layer 0, out block = wave
+  float dB[L > 1 ? L - 1 : 1];          // hidden bias of feature 32 (wave % 2) + lane % 32: positions of this lane half
+  float dwo[4 * NB];
+  float dbo;
+  __device__ __forceinline__ void zero() {
+#pragma unroll
+    for (int l = 0; l < (L > 1 ? L - 1 : 1); ++l) {
+#pragma unroll
+      for (int q = 0; q < 16; ++q) dW[l][q] = 0.0f;
+      dB[l] = 0.0f;
+    }
+    dW0 = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < 4 * NB; ++q) dwo[q] = 0.0f;
+    dbo = 0.0f;
+  }
+};
+
 template <int L, int NB>
 struct CoopAcc {
+  static constexpr bool kSplit = false;
   static constexpr int kW = (NB * NB + kBW - 1) / kBW;  // hidden-layer blocks owned per wavefront
   f4 dW[L > 1 ? L - 1 : 1][kW];                         // block q = wave * kW + j: (q / NB, q % NB)
   f4 dW0;                                               // layer 0, out block = wave (wave < NB)
@@ -763,6 +818,18 @@ struct CoopAcc {
                                                         // delta rows contracted with a row of ones (row 0)
   float dwo[4 * NB];                                    // per-lane partial output-weight sums
   float dbo;
+  __device__ __forceinline__ void zero() {
+#pragma unroll
+    for (int l = 0; l < (L > 1 ? L - 1 : 1); ++l) {
+#pragma unroll
+      for (int q = 0; q < kW; ++q) dW[l][q] = f4{0.f, 0.f, 0.f, 0.f};
+      dB[l] = f4{0.f, 0.f, 0.f, 0.f};
+    }
+    dW0 = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < 4 * NB; ++q) dwo[q] = 0.0f;
+    dbo = 0.0f;
+  }
 };
 
 // Operand stage geometry: rows of TP floats; with kPerm the rows of each group of 4
@@ -825,22 +892,23 @@ __device__ __forceinline__ f4 coop_block(const float* __restrict__ stage, int st
   return acc;
 }
 
-// writes the workgroup's gradient of one phase net into out[0 .. flat size)
-template <int L, int NB>
-__device__ void flush_coop(CoopAcc<L, NB>& G, FlatNet fn, float* __restrict__ red, float* __restrict__ out) {
-  using CA = CoopAcc<L, NB>;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
+// writes the gradient of one phase net that this group of kBW wavefronts has summed into out[0 .. flat size)
+template <int L, int NB, class Acc>
+__device__ void flush_coop(Acc& G, FlatNet fn, float* __restrict__ red, float* __restrict__ out) {
+  const int lane = threadIdx.x & 63, tid = threadIdx.x % kBT, wave = tid / 64;
   const int Hh = fn.Hh;
   const int P = 4 * Hh + (L - 1) * (Hh * Hh + Hh) + Hh + 1;  // parameters of this net
   const int base = fn.base;
-  for (int i = threadIdx.x; i < P; i += kBT) red[i] = 0.0f;
+  for (int i = tid; i < P; i += kBT) red[i] = 0.0f;
   __syncthreads();
   // row sums of the per-lane partials (every wavefront, no LDS)
 #pragma unroll
-  for (int q = 0; q < 4 * NB; ++q) {
-    G.dwo[q] = row16_sum(G.dwo[q]);
-  }
+  for (int q = 0; q < 4 * NB; ++q) G.dwo[q] = row16_sum(G.dwo[q]);
   G.dbo = row16_sum(G.dbo);
+  if constexpr (Acc::kSplit) {
+#pragma unroll
+    for (int l = 1; l < L; ++l) G.dB[l - 1] += __shfl_xor(G.dB[l - 1], 32, 64);
+  }
   // the delta of hidden layer l carries kTanhExp2Scale^(L-1-l) (weights packed times the factor): inv[l]
   // undoes it for layer l's weight and bias gradients (layer 0: its weights and bias, rows 0..3 of dW0)
   float inv[L];
@@ -852,15 +920,21 @@ __device__ void flush_coop(CoopAcc<L, NB>& G, FlatNet fn, float* __restrict__ re
     if (wave == w) {
 #pragma unroll
       for (int l = 1; l < L; ++l) {
+        auto put = [&](int in, int o, float v) {
+          if (in < Hh && o < Hh) red[fn.w(l) - base + in * Hh + o] = v * inv[l];
+        };
+        if constexpr (Acc::kSplit) {
 #pragma unroll
-        for (int j = 0; j < CA::kW; ++j) {
-          const int q = wave * CA::kW + j;
-          if (q < NB * NB) {
-            const int ib = q / NB, ob = q % NB;
+          for (int r = 0; r < 16; ++r)
+            put(32 * (wave / 2) + 8 * (r / 4) + 4 * (lane / 32) + r % 4, 32 * (wave % 2) + lane % 32, G.dW[l - 1][r]);
+        } else {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int in = 16 * ib + 4 * (lane / 16) + r, o = 16 * ob + (lane & 15);
-              if (in < Hh && o < Hh) red[fn.w(l) - base + in * Hh + o] = G.dW[l - 1][j][r] * inv[l];
+          for (int j = 0; j < Acc::kW; ++j) {
+            const int q = wave * Acc::kW + j;
+            if (q < NB * NB) {
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                put(16 * (q / NB) + 4 * (lane / 16) + r, 16 * (q % NB) + (lane & 15), G.dW[l - 1][j][r]);
             }
           }
         }
@@ -872,7 +946,12 @@ __device__ void flush_coop(CoopAcc<L, NB>& G, FlatNet fn, float* __restrict__ re
           if (row < 3 && o < Hh) red[fn.w(0) - base + row * Hh + o] = G.dW0[r] * inv[0];
           if (row == 3 && o < Hh) red[fn.b(0) - base + o] = G.dW0[r] * inv[0];
         }
-        if (lane < 16 && 16 * wave + lane < Hh) {
+        if constexpr (Acc::kSplit) {
+          if (wave < 2 && lane < 32 && 32 * wave + lane < Hh) {
+#pragma unroll
+            for (int l = 1; l < L; ++l) red[fn.b(l) - base + 32 * wave + lane] = G.dB[l - 1] * inv[l];
+          }
+        } else if (lane < 16 && 16 * wave + lane < Hh) {
 #pragma unroll
           for (int l = 1; l < L; ++l) red[fn.b(l) - base + 16 * wave + lane] = G.dB[l - 1][0] * inv[l];
         }
@@ -893,7 +972,7 @@ __device__ void flush_coop(CoopAcc<L, NB>& G, FlatNet fn, float* __restrict__ re
     }
     __syncthreads();
   }
-  for (int i = threadIdx.x; i < P; i += kBT) out[i] = red[i];
+  for (int i = tid; i < P; i += kBT) out[i] = red[i];
 }
 
 // c = W_l d_l of one tile (l >= 1, unscaled by the activation's derivative), d and c feature-major; W is the
@@ -943,20 +1022,20 @@ __device__ __forceinline__ void tile_backprop(const float* __restrict__ W, int l
   }
 }
 
-// kBf: W is the TransBf copy (W_l d_l as split bf16 products), the output weights come in wor and the
+// kBf: W is the TransBf copy (W_l d_l as split bf16 products), the output weights are at wor and the
 // stage rows are 16 floats with rotated row groups; else W is the float32 Packed copy (float32 MFMA) and
 // the stage rows are padded to kTP floats
 // prefetch() is called once per tile, as soon as act is no longer read (after the backprop through
 // layer 1, or at the start for L = 1), so that loads for the next tile can take its registers and their
 // latency overlaps the remaining contractions
 template <int L, int NB, bool kBf, class Prefetch>
-__device__ __forceinline__ void coop_backward(const float* __restrict__ W, const float (&wor)[4 * NB], float seed,
+__device__ __forceinline__ void coop_backward(const float* __restrict__ W, const float* __restrict__ wor, float seed,
                                               float xin, const float (&act)[L][4 * NB], float* __restrict__ stage,
                                               int stride_w, CoopAcc<L, NB>& G, Prefetch&& prefetch) {
   using PK = Packed<L, NB>;
   using CA = CoopAcc<L, NB>;
   using SG = std::conditional_t<kBf, StageRot, StagePad>;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x % kBT / 64;
   float* bufA = stage + wave * stride_w;
   float* bufD = bufA + stride_w / 2;
   // output layer
@@ -968,7 +1047,7 @@ __device__ __forceinline__ void coop_backward(const float* __restrict__ W, const
       const float a = act[L - 1][fb * 4 + r];
       float wo;
       if constexpr (kBf)
-        wo = wor[fb * 4 + r];
+        wo = wor[16 * fb + 4 * (lane / 16) + r];
       else
         wo = W[PK::wout() + 16 * fb + 4 * (lane / 16) + r];
       G.dwo[fb * 4 + r] = fmaf(a, seed, G.dwo[fb * 4 + r]);
@@ -1018,71 +1097,233 @@ __device__ __forceinline__ void coop_backward(const float* __restrict__ W, const
   }
 }
 
+// coop_backward for the 64-wide networks: every contraction as split-bf16 products.  Per layer each wavefront
+// stages the parts of its tile's deltas (split once, for this and for the back-propagation) and activations; after
+// the barrier wavefront w contracts block (w / 2, w % 2) of 32 x 32 over the group's kBW tiles.  The products of a round go
+// to a fresh accumulator that is then added to the running one: one rounding at the running sum's size per round.
+// Bound by the matrix and VALU cycles together (beside VALU work a bf16 MFMA still costs most of its own).  At 128^3
+// (star, last zoom level, 110 K tiles per batch): 619 -> 500 us against the same contraction in float32 MFMA, which
+// takes 2.7x the matrix cycles, during which the SIMD issues no VALU work at all.  Splitting with v_dot2 (7 instructions a
+// pair instead of 11): 2% slower, it does not run beside the MFMA either.
+template <int L, int NB, class Prefetch>
+__device__ __forceinline__ void split_backward(const float* __restrict__ W, const float* __restrict__ wor, float seed,
+                                               float xin, const float (&act)[L][4 * NB], float* __restrict__ stage,
+                                               SplitAcc<L, NB>& G, Prefetch&& prefetch) {
+  static_assert(NB == 4, "four 32x32 blocks for the kBW wavefronts of a group");
+  using SS = SplitStage<NB>;
+  using TB = TransBf<L, NB>;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x % kBT / 64;
+  uint16_t* const tiles = reinterpret_cast<uint16_t*>(stage);
+  uint16_t* const bufA = tiles + wave * SS::kTile;
+  uint16_t* const bufD = bufA + SS::kOperand;
+  const u4* __restrict__ wt = reinterpret_cast<const u4*>(W);
+  float d[4 * NB];
+#pragma unroll
+  for (int q = 0; q < 4 * NB; ++q) {
+    const float a = act[L - 1][q];
+    G.dwo[q] = fmaf(a, seed, G.dwo[q]);
+    d[q] = seed * wor[16 * (q / 4) + 4 * (lane / 16) + q % 4] * (1.0f - a * a);
+  }
+  if (lane < 16) G.dbo += seed;
+  if constexpr (L == 1) prefetch();
+#pragma unroll
+  for (int l = L - 1; l >= 0; --l) {
+    f4 c[NB];
+#pragma unroll
+    for (int ib = 0; ib < NB; ++ib) c[ib] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int cc = 0; cc < TB::NC; ++cc) {
+      u4 h, m, lo;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int q = 8 * cc + 2 * u;
+        uint32_t a0, a1, a2;
+        bf_split_pair(d[q], d[q + 1], a0, a1, a2);
+        h[u] = a0;
+        m[u] = a1;
+        lo[u] = a2;
+      }
+      split_stage<NB>(bufD, cc, h, m, lo);
+      if (l > 0) {
+        // d_{l-1} = (W_l d_l) * (1 - a_{l-1}^2), before the barrier: a wavefront that arrives early does this
+        // matrix work while it waits
+        u4 w[3];
+        bf_chunk<NB, TB::NC, false>(wt, [&](int ib, int ch) { return TB::set(l, ib, ch, 0); }, cc, h, m, lo, w, c);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int q = 8 * cc + 2 * u;
+          uint32_t a0, a1, a2;
+          bf_split_pair(act[l - 1][q], act[l - 1][q + 1], a0, a1, a2);
+          h[u] = a0;
+          m[u] = a1;
+          lo[u] = a2;
+        }
+        split_stage<NB>(bufA, cc, h, m, lo);
+      }
+    }
+    if (l > 0) {
+#pragma unroll
+      for (int q = 0; q < 4 * NB; ++q) {
+        const float a = act[l - 1][q];
+        d[q] = c[q / 4][q % 4] * (1.0f - a * a);
+      }
+      if (l == 1) prefetch();
+    } else {
+      uint32_t h, m, lo;
+      bf_split_pair(xin, 0.0f, h, m, lo);
+      uint16_t* in = bufA + (lane & 15) * 4 + (lane >> 4);
+      in[0] = (uint16_t)h;
+      in[SS::kInPart] = (uint16_t)m;
+      in[2 * SS::kInPart] = (uint16_t)lo;
+    }
+    __syncthreads();
+    // lane group kg, lane i of a group: in a 32x32x16 operand block kg % 2 of its two, positions 8 (kg / 2) .. + 7
+    const int kg = lane >> 4, i = lane & 15;
+    __builtin_amdgcn_s_setprio(1);  // before the other group's staging (1%)
+    if (l > 0) {
+      const int p0 = 8 * (kg >> 1) + (i >> 2);
+      const int lo = SS::unit(kg & 1, i & 3, p0), hi = SS::unit(kg & 1, i & 3, p0 + 4);
+      f16v t;
+      float tb = 0.0f;  // sum over the positions of this lane's feature of the deltas
+#pragma unroll
+      for (int q = 0; q < 16; ++q) t[q] = 0.0f;
+#pragma unroll
+      for (int s = 0; s < kBW; ++s) {
+        const uint16_t* A = tiles + s * SS::kTile;
+        const uint16_t* D = A + SS::kOperand;
+        u4 a[3], b[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+          const uint16_t* ap = A + p * SS::kPart + 512 * (wave / 2);
+          const uint16_t* bp = D + p * SS::kPart + 512 * (wave % 2);
+          a[p] = tr_read8(ap + lo, ap + hi);
+          b[p] = tr_read8(bp + lo, bp + hi);
+        }
+#pragma unroll
+        for (int p = 2; p >= 0; --p)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const uint32_t pair = b[p][u];
+            tb = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf2, pair), bf2{(__bf16)1.0f, (__bf16)1.0f}, tb, false);
+          }
+        t = mfma_bf32(a[2], b[0], t);
+        t = mfma_bf32(a[1], b[1], t);
+        t = mfma_bf32(a[0], b[2], t);
+        t = mfma_bf32(a[1], b[0], t);
+        t = mfma_bf32(a[0], b[1], t);
+        t = mfma_bf32(a[0], b[0], t);
+        __builtin_amdgcn_sched_barrier(0);  // one tile's operands at a time
+      }
+#pragma unroll
+      for (int q = 0; q < 16; ++q) G.dW[l - 1][q] += t[q];
+      G.dB[l - 1] += tb;
+    } else {
+      // layer 0: rows x, y, z, 1 (repeated to 16) against out block `wave`; K = 32: two tiles per product
+      const int p0 = 8 * (kg & 1) + (i >> 2);
+      const int lo = SS::unit(wave, i & 3, p0), hi = SS::unit(wave, i & 3, p0 + 4);
+      f4 t = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < kBW; s += 2) {
+        const uint16_t* A = tiles + (s + (kg >> 1)) * SS::kTile;
+        const uint16_t* D = A + SS::kOperand;
+        u4 a[3], b[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+          const uint16_t* ap = A + p * SS::kInPart + 4 * p0;
+          const uint16_t* bp = D + p * SS::kPart;
+          a[p] = tr_read8(ap, ap + 16);
+          b[p] = tr_read8(bp + lo, bp + hi);
+        }
+        t = bf6(a, b[0], b[1], b[2], t);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) G.dW0[r] += t[r];
+    }
+    __builtin_amdgcn_s_setprio(0);
+    __syncthreads();  // operands consumed: the buffers may be restaged
+  }
+}
+
+// Groups of kBW wavefronts per backward workgroup, each with tiles, stage and partial rows of its own.  With a
+// 64-wide network a workgroup has two, which share the back-propagation weights (48 KB; with two stages of 54 KB
+// one workgroup fills a CU's LDS); the second runs one barrier behind the first, so that between any two barriers one group stages
+// and back-propagates (VALU) while the other contracts (matrix cores, LDS).  The recomputing variant, which also holds the
+// forward copy, has room for one; a group's tiles and sums are the same either way.
+template <int NBm, int NBp, bool kStored>
+constexpr int bwd_groups() {
+  return kStored && (NBm == 4 || NBp == 4) ? 2 : 1;
+}
+
 // LDS of the backward kernel for one phase net (floats): its backprop weights (the TransBf copy from two
 // 16-wide blocks on, the float32 Packed copy below), with kStored false the forward pass's split-bf16 copy
-// (PackedBf, where the forward pass uses one), then the operand stage of the kBW wavefronts (rows of 16
-// floats, rotated, with TransBf; of kTP floats with Packed).  3x64 with kStored: 48 KB + 32 KB = 80 KB,
-// two workgroups per CU.
-template <int L, int NB, bool kStored>
+// (PackedBf, where the forward pass uses one), then the operand stage of the kBW wavefronts of every group
+// (SplitStage for 64-wide networks; else rows of 16 floats, rotated, with TransBf, of kTP floats with Packed).
+template <int L, int NB, bool kStored, int kGroups>
 struct BwdPhase {
   static constexpr bool kBf = FwdPack<L, NB>::kBf;
+  static constexpr bool kSplit = NB == 4;
   static constexpr int wr() { return ((kBf ? TransBf<L, NB>::size() : Packed<L, NB>::size()) + 3) & ~3; }
+  static constexpr int edges() { return kBf ? 80 * NB : 0; }  // pack_edges
   static constexpr int fp() { return (!kStored && kBf) ? ((PackedBf<L, NB>::size() + 3) & ~3) : 0; }
-  static constexpr int stride() { return 2 * 16 * NB * (kBf ? StageRot::kTPs : StagePad::kTPs); }
-  static constexpr int floats() { return wr() + fp() + kBW * stride(); }
+  static constexpr int stride() {
+    return kSplit ? SplitStage<NB>::floats() : 2 * 16 * NB * (kBf ? StageRot::kTPs : StagePad::kTPs);
+  }
+  static constexpr int floats() { return wr() + edges() + fp() + kGroups * kBW * stride(); }
 };
 template <int Lm, int NBm, int Lp, int NBp, bool kStored>
 struct BwdLds {
-  static constexpr int kP = BwdPhase<Lp, NBp, kStored>::floats(), kM = BwdPhase<Lm, NBm, kStored>::floats();
-  static constexpr int floats() { return kP > kM ? kP : kM; }
+  static constexpr int kGroups = bwd_groups<NBm, NBp, kStored>();
+  static constexpr int kP = BwdPhase<Lp, NBp, kStored, kGroups>::floats(),
+                       kM = BwdPhase<Lm, NBm, kStored, kGroups>::floats();
+  // the flush holds each group's gradient of one net (of the widest width the shape takes)
+  static constexpr int net(int L, int H) { return 4 * H + (L - 1) * (H * H + H) + H + 1; }
+  static constexpr int kRed = kGroups * (net(Lp, 16 * NBp) > net(Lm, 16 * NBm) ? net(Lp, 16 * NBp) : net(Lm, 16 * NBm));
+  static constexpr int kMax = kP > kM ? kP : kM;
+  static constexpr int floats() { return kMax > kRed ? kMax : kRed; }
 };
 
 // kStored: the activations of every tile come from the forward kernel (act_in, act_f4 f4s per lane and
 // tile, + tiles first); else each wavefront recomputes them with the forward kernel's arithmetic (the
-// same split-bf16 or float32 pass, so both variants give the same bits)
+// same split-bf16 or float32 pass, so both variants give the same bits).  Groups (blockIdx kGroups + group)
+// [0, ngrp_p) take the + tiles, the rest of the ngrp the - tiles; both counts are multiples of kGroups.
 template <int Lm, int NBm, int Lp, int NBp, bool kStored>
-__global__ __launch_bounds__(kBT, 2) void mfma_bwd_kernel(MfmaTileArgs T, const float* __restrict__ params, int Hm, int Hp,
-                                                       int64_t e0, int64_t np_, int64_t nm_,
-                                                       const float* __restrict__ seed_item, float* __restrict__ gpart,
-                                                       int nblk_p, int stride, const f4* __restrict__ act_in,
-                                                       int act_f4) {
+__global__ __launch_bounds__((kBT * bwd_groups<NBm, NBp, kStored>()), 2) void mfma_bwd_kernel(
+    MfmaTileArgs T, const float* __restrict__ params, int Hm, int Hp, int64_t e0, int64_t np_, int64_t nm_,
+    const float* __restrict__ seed_item, float* __restrict__ gpart, int ngrp_p, int stride,
+    const f4* __restrict__ act_in, int act_f4) {
   extern __shared__ __align__(16) float lds[];
-  const int wave = threadIdx.x / 64, lane = threadIdx.x & 63;
-  const bool plus = (int)blockIdx.x < nblk_p;
+  constexpr int kGroups = bwd_groups<NBm, NBp, kStored>();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x % kBT / 64;
+  const int group = kGroups > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kBT) : 0;
+  const int grp = (int)blockIdx.x * kGroups + group, ngrp = (int)gridDim.x * kGroups;
+  const bool plus = (int)blockIdx.x * kGroups < ngrp_p;
   const int PPp = 4 * Hp + (Lp - 1) * (Hp * Hp + Hp) + Hp + 1;
   const int64_t ntp = (np_ + 15) / 16;
   const int64_t ntiles = plus ? (np_ + 15) / 16 : (nm_ + 15) / 16;
-  const int nblk = plus ? nblk_p : (int)gridDim.x - nblk_p;
-  const int bid = plus ? (int)blockIdx.x : (int)blockIdx.x - nblk_p;
+  const int nblk = plus ? ngrp_p : ngrp - ngrp_p;
+  const int bid = plus ? grp : grp - ngrp_p;
   const int64_t eb = plus ? e0 : e0 + np_;
   const int64_t ee = plus ? e0 + np_ : e0 + np_ + nm_;
-  float* out = gpart + (int64_t)blockIdx.x * stride;
+  float* out = gpart + (int64_t)grp * stride;
   auto run = [&](auto tagL, auto tagNB, FlatNet fn) {
     constexpr int L = decltype(tagL)::value;
     constexpr int NB = decltype(tagNB)::value;
-    using CA = CoopAcc<L, NB>;
-    using BP = BwdPhase<L, NB, kStored>;
-    // the forward copy and the operand stage start on 16-byte boundaries after the backprop weights
-    float* fwdW = lds + BP::wr();
-    float* stage = lds + BP::wr() + BP::fp();
+    using BP = BwdPhase<L, NB, kStored, kGroups>;
+    using Acc = std::conditional_t<BP::kSplit, SplitAcc<L, NB>, CoopAcc<L, NB>>;
+    // the forward copy and the operand stages start on 16-byte boundaries after the backprop weights
+    float* edges = lds + BP::wr();
+    float* fwdW = edges + BP::edges();
+    float* stage = fwdW + BP::fp() + group * kBW * BP::stride();
     if constexpr (BP::kBf) {
       pack_trans_bf<L, NB>(params, fn, lds);
+      pack_edges<NB>(params, fn, edges);
       if constexpr (!kStored) pack_weights_bf<L, NB>(params, fn, fwdW);
     } else {
       pack_weights<L, NB>(params, fn, lds);
     }
     __syncthreads();
-    CA G;
-#pragma unroll
-    for (int l = 0; l < (L > 1 ? L - 1 : 1); ++l)
-#pragma unroll
-      for (int q = 0; q < CA::kW; ++q) G.dW[l][q] = f4{0.f, 0.f, 0.f, 0.f};
-    G.dW0 = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int l = 0; l < (L > 1 ? L - 1 : 1); ++l) G.dB[l] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int q = 0; q < 4 * NB; ++q) G.dwo[q] = 0.0f;
-    G.dbo = 0.0f;
+    Acc G;
+    G.zero();
     // every wavefront runs the same number of rounds (the barriers inside);
     // tiles past the end carry no entries (zero seeds, zero inputs)
     const int64_t per_round = (int64_t)nblk * kBW;
@@ -1095,22 +1336,16 @@ __global__ __launch_bounds__(kBT, 2) void mfma_bwd_kernel(MfmaTileArgs T, const 
     float xin_next = item_input(T, item_of(0), ee, kq);
     float seed_next = seed_of(item_of(0));
     // the stored activations of a round's tile (layers 1..L-1), loaded for round rd + 1 inside round rd
-    // once its activations are dead
+    // once its activations are dead.  Past the phase's tiles the last one's are read again (finite, seeds zero).
     float act_n[L][4 * NB];
     auto load_round = [&](int64_t rd) {
       if constexpr (kStored) {
-        const int64_t tile = (rd * nblk + bid) * kBW + wave;
-        if (tile < ntiles) {
-          load_act<L, NB>(act_in + ((plus ? tile : ntp + tile) * act_f4) * 64 + lane, act_n);
-        } else {
-#pragma unroll
-          for (int l = 1; l < L; ++l)
-#pragma unroll
-            for (int q = 0; q < 4 * NB; ++q) act_n[l][q] = 0.0f;
-        }
+        const int64_t tile = min((rd * nblk + bid) * kBW + wave, ntiles - 1);
+        load_act<L, NB>(act_in + ((plus ? tile : ntp + tile) * act_f4) * 64 + lane, act_n);
       }
     };
     load_round(0);
+    if (kGroups > 1 && BP::kSplit && group == 1) __syncthreads();  // one barrier behind the first group
     for (int64_t rd = 0; rd < rounds; ++rd) {
       const float xin = xin_next, seed = seed_next;
       if (rd + 1 < rounds) {
@@ -1119,36 +1354,31 @@ __global__ __launch_bounds__(kBT, 2) void mfma_bwd_kernel(MfmaTileArgs T, const 
         seed_next = seed_of(nx);
       }
       float act[L][4 * NB];
-      // with TransBf: layer 0's operands and the output weights of this lane, loaded per round (cached
-      // reads of the parameter vector; held across rounds they would spill)
-      float w0r[NB], wor[4 * NB];
-      if constexpr (BP::kBf) lane_weights<NB>(params, fn, w0r, wor);
       if constexpr (kStored) {
 #pragma unroll
         for (int l = 1; l < L; ++l)
 #pragma unroll
           for (int q = 0; q < 4 * NB; ++q) act[l][q] = act_n[l][q];
-        if constexpr (BP::kBf)
-          tile_layer0_regs<L, NB>(w0r, xin, act);
-        else
-          tile_layer0<L, NB>(lds, xin, act);
+        tile_layer0<L, NB>(BP::kBf ? edges : lds, xin, act);
       } else if constexpr (BP::kBf) {
         tile_forward_bf<L, NB>(fwdW, xin, act);
       } else {
         tile_forward<L, NB>(lds, xin, act);
       }
-      coop_backward<L, NB, BP::kBf>(lds, wor, seed, xin, act, stage, BP::stride(), G, [&] {
-        if (rd + 1 < rounds) load_round(rd + 1);
-      });
+      auto prefetch = [&] { load_round(rd + 1); };
+      if constexpr (BP::kSplit)
+        split_backward<L, NB>(lds, edges + 64 * NB, seed, xin, act, stage, G, prefetch);
+      else
+        coop_backward<L, NB, BP::kBf>(lds, edges + 64 * NB, seed, xin, act, stage, BP::stride(), G, prefetch);
     }
+    if (kGroups > 1 && BP::kSplit && group == 0) __syncthreads();
     __syncthreads();  // all waves done with the packed weights: reuse LDS for the reduction
-    flush_coop<L, NB>(G, fn, lds, out);
+    flush_coop<L, NB>(G, fn, lds + group * stride, out);
   };
   if (plus)
     run(std::integral_constant<int, Lp>{}, std::integral_constant<int, NBp>{}, FlatNet{Hp, Lp, 0});
   else
     run(std::integral_constant<int, Lm>{}, std::integral_constant<int, NBm>{}, FlatNet{Hm, Lm, PPp});
-  (void)lane;
 }
 
 // ---- kernel 4/5: reduction of gradient partials and optimizer -------------------
@@ -1464,7 +1694,7 @@ static int act_f4_of(const dips_net_t* n) {
 static int64_t mfma_base_floats(const dips_net_t* n, int64_t max_rows, int64_t max_nnz) {
   const int P = net_params(n->Lm, n->Hm) + net_params(n->Lp, n->Hp);
   const int stride = std::max(net_params(n->Lm, n->Hm), net_params(n->Lp, n->Hp));
-  return max_nnz + max_rows + (int64_t)kMfmaBwdBlocks * stride + P + 64;
+  return max_nnz + max_rows + (int64_t)kMfmaBwdGroups * stride + P + 64;
 }
 
 // ... plus, 256-byte aligned, the hidden activations of every forward tile (at most max_nnz / 16 + 2 tiles:
@@ -1562,7 +1792,7 @@ int mfma_step(const dips_grid_t* g, const dips_records_t* rec, const dips_mfma_b
   float* u = work;  // indexed by item - i0
   float* r = u + nent;
   float* gpart = r + nrows;
-  float* gvec = gpart + (int64_t)kMfmaBwdBlocks * stride;
+  float* gvec = gpart + (int64_t)kMfmaBwdGroups * stride;
   int32_t* count_snap = reinterpret_cast<int32_t*>(gvec + P);
   if ((int64_t)(gvec + P + 1 - work) > work_floats) {
     set_error("dips_mfma_train_step: workspace too small");
@@ -1601,41 +1831,44 @@ int mfma_step(const dips_grid_t* g, const dips_records_t* rec, const dips_mfma_b
   const bool stored = act_off + (ntp + ntm) * act_f4 * 256 <= work_floats;
   f4* act = stored ? reinterpret_cast<f4*>(work + act_off) : nullptr;
   // workgroups split by phase in proportion to the tiles (each at least 1 if it has tiles)
-  auto split = [&](int total, int& p, int& m) {
-    p = (ntp > 0) ? (int)std::max<int64_t>(1, (int64_t)((double)total * ntp / std::max<int64_t>(1, ntp + ntm))) : 0;
-    m = (ntm > 0) ? std::max(1, total - p) : 0;
-    if (p + m > total) p = total - m;
+  // (in multiples of unit, which divides total)
+  auto split = [&](int total, int unit, int& p, int& m) {
+    const int t = total / unit;
+    p = (ntp > 0) ? (int)std::max<int64_t>(1, (int64_t)((double)t * ntp / std::max<int64_t>(1, ntp + ntm))) : 0;
+    m = (ntm > 0) ? std::max(1, t - p) : 0;
+    if (p + m > t) p = t - m;
+    p *= unit;
+    m *= unit;
   };
   int nbp, nbm, nfp, nfm;
-  split(kMfmaBwdBlocks, nbp, nbm);
+  // groups of the backward, in pairs whichever variant runs: the same tiles and partial rows for both
+  split(kMfmaBwdGroups, (b == 4 || d == 4) ? 2 : 1, nbp, nbm);
   bool launched = false;
 #define X(A, B, C, D)                                                                                              \
   if (!launched && a == A && b == B && c == C && d == D) {                                                      \
     launched = true;                                                                                               \
     constexpr int PKF = FwdPack<C, D>::size() > FwdPack<A, B>::size() ? FwdPack<C, D>::size() : FwdPack<A, B>::size(); \
     const size_t lds_f = sizeof(float) * PKF;                                                                      \
-    const size_t red_b = sizeof(float) * std::max(PPp, PPm);                                                       \
-    const size_t bwd_lds = std::max(sizeof(float) * (stored ? BwdLds<A, B, C, D, true>::floats()                   \
-                                                            : BwdLds<A, B, C, D, false>::floats()), red_b);        \
+    const size_t bwd_lds = sizeof(float) * (stored ? BwdLds<A, B, C, D, true>::floats()                            \
+                                                   : BwdLds<A, B, C, D, false>::floats());                         \
     if (bwd_lds > 160 * 1024 || lds_f > 160 * 1024) {                                                              \
       set_error("dips_mfma_train_step: network too large for the LDS of one workgroup");                            \
       return DIPS_EUNSUPPORTED;                                                                                    \
     }                                                                                                              \
     /* LDS limits set once per instantiation (for its widest networks), so that a step is launches only */      \
     static const bool attrs_set = [] {                                                                             \
-      const size_t red_max = sizeof(float) * std::max(net_params(C, 16 * D), net_params(A, 16 * B));             \
       hipFuncSetAttribute((const void*)mfma_fwd_kernel<A, B, C, D>, hipFuncAttributeMaxDynamicSharedMemorySize,    \
                           (int)(sizeof(float) * PKF));                                                             \
       hipFuncSetAttribute((const void*)mfma_bwd_kernel<A, B, C, D, true>,                                          \
                           hipFuncAttributeMaxDynamicSharedMemorySize,                                              \
-                          (int)std::max(sizeof(float) * BwdLds<A, B, C, D, true>::floats(), red_max));             \
+                          (int)(sizeof(float) * BwdLds<A, B, C, D, true>::floats()));                              \
       hipFuncSetAttribute((const void*)mfma_bwd_kernel<A, B, C, D, false>,                                         \
                           hipFuncAttributeMaxDynamicSharedMemorySize,                                              \
-                          (int)std::max(sizeof(float) * BwdLds<A, B, C, D, false>::floats(), red_max));            \
+                          (int)(sizeof(float) * BwdLds<A, B, C, D, false>::floats()));                             \
       return true;                                                                                                 \
     }();                                                                                                           \
     (void)attrs_set;                                                                                               \
-    split(resident_blocks((const void*)mfma_fwd_kernel<A, B, C, D>, kFT, lds_f, kMfmaFwdBlocks), nfp, nfm);       \
+    split(resident_blocks((const void*)mfma_fwd_kernel<A, B, C, D>, kFT, lds_f, kMfmaFwdBlocks), 1, nfp, nfm);       \
     if (nfp + nfm > 0)                                                                                             \
       hipLaunchKernelGGL((mfma_fwd_kernel<A, B, C, D>), dim3(nfp + nfm), dim3(kFT), lds_f, st, T, params, Hm, Hp,   \
                          i0, ip, im, u, nfp, act, act_f4);                                                         \
@@ -1645,7 +1878,8 @@ int mfma_step(const dips_grid_t* g, const dips_records_t* rec, const dips_mfma_b
       hipLaunchKernelGGL(mfma_seed_kernel, dim3(xcd_grid((ip + im + 255) / 256)), dim3(256), 0, st, T, i0,          \
                          ip + im, bt->row_begin, r, u);                                                            \
     if (nbp + nbm > 0 && stored)                                                                                   \
-      hipLaunchKernelGGL((mfma_bwd_kernel<A, B, C, D, true>), dim3(nbp + nbm), dim3(kBT), bwd_lds, st, T,           \
+      hipLaunchKernelGGL((mfma_bwd_kernel<A, B, C, D, true>), dim3((nbp + nbm) / BwdLds<A, B, C, D, true>::kGroups), \
+                         dim3(kBT * BwdLds<A, B, C, D, true>::kGroups), bwd_lds, st, T,                            \
                          params, Hm, Hp, i0, ip, im, u, gpart, nbp, stride, act, act_f4);                          \
     if (nbp + nbm > 0 && !stored)                                                                                  \
       hipLaunchKernelGGL((mfma_bwd_kernel<A, B, C, D, false>), dim3(nbp + nbm), dim3(kBT), bwd_lds, st, T,          \
