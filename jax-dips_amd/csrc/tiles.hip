@@ -39,8 +39,6 @@ namespace dips {
 
 constexpr int kTileCap = 64;                          // entries and rows of a packed tile
 constexpr int kMaxTileBlocks = 256;                   // one workgroup per CU
-constexpr int kBlocksPerLane = kMaxTileBlocks / DIPS_WAVE;
-constexpr int kReduceChunk = 8;                       // parameters per wavefront per load round
 constexpr int kLdsStride = 68;                        // floats per staged operand row: 64 entries + 4
 constexpr int kStageFloats = 2 * 16 * kLdsStride;     // A and B operand stacks of one wavefront
 
@@ -97,15 +95,27 @@ constexpr uint32_t kSlotUsed = 1u << 13;
 
 __device__ __forceinline__ int64_t clamp64(int64_t v, int64_t lo, int64_t hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
-// The last workgroup of a fused launch: reduce the parameter-major partial rows
-// (partial[p * nblk + b], nblk <= kMaxTileBlocks) in a fixed order and apply
-// the optimizer to params / m / v.
+// four consecutive floats at 4-byte alignment (rows have odd lengths): one 16-byte load
+typedef float row4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef const __attribute__((address_space(1))) row4 global_row4;
+
+// Reduce the partial rows (partial[b * kStride + p], b < nblk <= kMaxTileBlocks) in a fixed order, in float64,
+// and apply the optimizer to params / m / v; one workgroup.
+// A lane owns four neighbouring parameters (16-byte loads of a row) and a group of wavefronts every kGroups-th row;
+// the groups' sums meet in LDS and are added in order.  The kernel is a latency chain (rows -> norm ->
+// update) on one CU; with a wavefront's lanes over the rows instead, the float64 exchange between the lanes of every
+// parameter was most of it: 20.7 -> 7.2 us (32 rows of 707), 11.7 -> 8.0 us (256 of 420), 6.3 -> 5.9 us (256 of 168).
+// kGroups depends on the shape only, so that every launch form adds in the same order.
 template <int kStride, int kTileWaves>
 __device__ void tile_reduce_apply(const float* partial, int nblk, const FusedOpt& fo, float* params) {
   constexpr int kTileThreads = kTileWaves * DIPS_WAVE;
   constexpr int PT = kStride - 1;
-  constexpr int kPer = (kStride + kTileWaves - 1) / kTileWaves;  // parameters per wavefront
-  constexpr int kOwn = (PT + kTileThreads - 1) / kTileThreads;   // parameters updated per thread
+  constexpr int kOwn = (PT + kTileThreads - 1) / kTileThreads;        // parameters updated per thread
+  constexpr int kRowWaves = (kStride + 4 * DIPS_WAVE - 1) / (4 * DIPS_WAVE);  // wavefronts of a row
+  constexpr int kGroups = 16 / kRowWaves;
+  constexpr int kTeams = kTileWaves / kRowWaves;  // groups at work at once
+  static_assert(kStride >= 4 && kRowWaves <= 8 && kRowWaves <= kTileWaves, "partial row width");
+  __shared__ double gsum[kGroups][kStride];
   __shared__ float gsh[kStride];
   __shared__ double dred[kTileWaves];
   __shared__ float sched[3];
@@ -113,9 +123,8 @@ __device__ void tile_reduce_apply(const float* partial, int nblk, const FusedOpt
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / DIPS_WAVE);
   // every global read is issued up front so that their latencies overlap: the
   // optimizer state of the parameters this thread updates, the step counter,
-  // and the partial rows (plain, unconditional index-clamped loads after the
-  // caller's acquire; each wavefront reduces a set of parameters, its lanes
-  // stride over the workgroups)
+  // and the partial rows (plain loads after the caller's acquire, the last column's lanes clamped to the row's
+  // end: they repeat its sums)
   float pv[kOwn], mv[kOwn], vv[kOwn];
 #pragma unroll
   for (int q = 0; q < kOwn; ++q) {
@@ -126,43 +135,38 @@ __device__ void tile_reduce_apply(const float* partial, int nblk, const FusedOpt
     vv[q] = gld(fo.v, pc);
   }
   const int c = gld(fo.count, 0);
-  if (wave == 0) {
-    // step-dependent scalars, computed once (powf is long) while the partial
-    // rows are loaded by the other wavefronts
-    const float t1 = (float)(c + 1);
-    if (lane == 0) {
-      sched[0] = schedule_lr(fo.opt, c);
-      sched[1] = 1.0f - powf(0.9f, t1);
-      sched[2] = 1.0f - powf(0.999f, t1);
+  const int col = min(4 * (wave % kRowWaves * DIPS_WAVE + lane), kStride - 4);
+  for (int g = wave / kRowWaves; g < kGroups && wave < kTeams * kRowWaves; g += kTeams) {
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    constexpr int kChunk = 16;  // rows in flight
+    for (int b0 = g; b0 < nblk; b0 += kChunk * kGroups) {
+      row4 v[kChunk];
+#pragma unroll
+      for (int j = 0; j < kChunk; ++j)
+        v[j] = *(global_row4*)(partial + (int64_t)min(b0 + j * kGroups, nblk - 1) * kStride + col);
+#pragma unroll
+      for (int j = 0; j < kChunk; ++j)
+        if (b0 + j * kGroups < nblk) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[i] += (double)v[j][i];
+        }
     }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) gsum[g][col + i] = acc[i];
   }
-  // one round of loads when the wavefront's parameters fit (<= 32 per wavefront: the preconditioned
-  // networks' 420 parameters load in one round instead of four), else rounds of 16 (the 707 of the 2x16
-  // networks: three); the summation order is the same
-  constexpr int kChunk = kPer <= 4 * kReduceChunk ? kPer : 2 * kReduceChunk;
-  for (int q0 = 0; q0 < kPer; q0 += kChunk) {
-    float vals[kChunk][kBlocksPerLane];
+  __syncthreads();
+  if (wave == kTileWaves - 1 && lane == 0) {
+    // step-dependent scalars, computed once (powf is long) beside the other wavefronts' sums
+    const float t1 = (float)(c + 1);
+    sched[0] = schedule_lr(fo.opt, c);
+    sched[1] = 1.0f - powf(0.9f, t1);
+    sched[2] = 1.0f - powf(0.999f, t1);
+  }
+  for (int p = threadIdx.x; p < kStride; p += kTileThreads) {
+    double acc = 0.0;
 #pragma unroll
-    for (int qq = 0; qq < kChunk; ++qq) {
-      const int p = wave + (q0 + qq) * kTileWaves;
-#pragma unroll
-      for (int i = 0; i < kBlocksPerLane; ++i) {
-        const int b = lane + i * DIPS_WAVE;
-        const int pc = p < kStride ? p : kStride - 1;
-        const int bc = b < nblk ? b : nblk - 1;
-        const float val = gld(partial, (int64_t)pc * nblk + bc);
-        vals[qq][i] = b < nblk ? val : 0.0f;  // p >= kStride: a duplicate, never stored
-      }
-    }
-#pragma unroll
-    for (int qq = 0; qq < kChunk; ++qq) {
-      const int p = wave + (q0 + qq) * kTileWaves;
-      double acc = 0.0;
-#pragma unroll
-      for (int i = 0; i < kBlocksPerLane; ++i) acc += (double)vals[qq][i];
-      acc = dips_wave_sum_d(acc);
-      if (lane == 0 && p < kStride) gsh[p] = (float)(acc * (double)fo.inv_b);
-    }
+    for (int g = 0; g < kGroups; ++g) acc += gsum[g][p];
+    gsh[p] = (float)(acc * (double)fo.inv_b);
   }
   __syncthreads();
   double sq = 0.0;
@@ -193,8 +197,7 @@ __device__ void tile_reduce_apply(const float* partial, int nblk, const FusedOpt
   }
 }
 
-// Reduction of the parameter-major partial rows of a tile_step_kernel launch
-// (kOut = 1) and the optimizer, as a kernel of its own: the kernel boundary
+// Reduction of the partial rows of a tile_step_kernel launch and the optimizer, as a kernel of its own: the kernel boundary
 // orders the partial rows before their reads.
 template <int kStride>
 __global__ __launch_bounds__(1024) void tile_apply_kernel(const float* partial, int nblk, FusedOpt fo,
@@ -590,9 +593,7 @@ struct TileCfg {
   static constexpr size_t kLdsBytes = sizeof(float) * kStageFloats * kWaves;
 };
 
-// kOut: 0 = block-major partial rows (for dips_opt_step), 1 = parameter-major
-// rows (for tile_apply_kernel), 2 = parameter-major rows and the fused
-// last-workgroup reduction + optimizer.
+// kFused: the last workgroup also reduces the partial rows and applies the optimizer.
 //
 // With a preconditioner (PC1 > 0) the row's residual is r = P * r0 with
 // P = 0.5 + s*sigmoid(MLP(cell coefficients)) evaluated at the row's last
@@ -601,9 +602,8 @@ struct TileCfg {
 // receive r * r0 * dP/dtheta.
 //
 // The body of one workgroup: block blk of nblk workgroups over the tiles of
-// a.  Writes the workgroup's partial row (kOut 0: partial[blk * stride + p],
-// else partial[p * nblk + blk]).
-template <int Lm, int Hm, int Lp, int Hp, bool kGrad, int kOut, int PC1, int PC2, int Act>
+// a.  Writes the workgroup's partial row partial[blk * stride + p].
+template <int Lm, int Hm, int Lp, int Hp, bool kGrad, int PC1, int PC2, int Act>
 __device__ __forceinline__ void tile_step_body(const TileStepArgs& a, float* params, float* __restrict__ partial,
                                                int blk, int nblk) {
   constexpr int kTileThreads = TileCfg<Lm, Hm, Lp, Hp, PC1>::kThreads;
@@ -851,10 +851,7 @@ __device__ __forceinline__ void tile_step_body(const TileStepArgs& a, float* par
 #pragma unroll
       for (int w = 0; w < kTileWaves; ++w) s += red[w * stride + p];
     }
-    if (kOut == 0)
-      gst(partial, (int64_t)blk * stride + p, s);
-    else
-      gst(partial, (int64_t)p * nblk + blk, s);
+    gst(partial, (int64_t)blk * stride + p, s);
   }
 }
 
@@ -864,14 +861,14 @@ constexpr int tile_stride() {
          (PC1 > 0 ? Precond<(PC1 > 0 ? PC1 : 1), PC2>::size() : 0) + 1;
 }
 
-template <int Lm, int Hm, int Lp, int Hp, bool kGrad, int kOut, int PC1 = 0, int PC2 = 0, int Act = kActTanh>
+template <int Lm, int Hm, int Lp, int Hp, bool kGrad, bool kFused, int PC1 = 0, int PC2 = 0, int Act = kActTanh>
 __global__ __launch_bounds__((TileCfg<Lm, Hm, Lp, Hp, PC1>::kThreads)) void tile_step_kernel(
     TileStepArgs a, float* params, float* __restrict__ partial, FusedOpt fo) {
   constexpr int kTileWaves = TileCfg<Lm, Hm, Lp, Hp, PC1>::kWaves;
   constexpr int stride = tile_stride<Lm, Hm, Lp, Hp, PC1, PC2>();
   const int nblk = (int)gridDim.x;
-  tile_step_body<Lm, Hm, Lp, Hp, kGrad, kOut, PC1, PC2, Act>(a, params, partial, (int)blockIdx.x, nblk);
-  if (kOut != 2) return;
+  tile_step_body<Lm, Hm, Lp, Hp, kGrad, PC1, PC2, Act>(a, params, partial, (int)blockIdx.x, nblk);
+  if (!kFused) return;
 
   // One thread per workgroup fences and counts: the barrier completes the
   // workgroup's partial stores, the agent-scope release makes them visible to
@@ -925,16 +922,16 @@ static void tile_launch_shape(const TileStepArgs& a, float* params, float* parti
   hipLaunchKernelGGL((tile_step_kernel<Lm, Hm, Lp, Hp, G, F, PC1, PC2, Act>), grid, block, lds, st, a, params,      \
                      partial, fo)
   if (mode == 2) {
-    DIPS_TILE_LAUNCH(true, 2);
+    DIPS_TILE_LAUNCH(true, true);
   } else if (mode == 3) {
-    DIPS_TILE_LAUNCH(true, 1);
+    DIPS_TILE_LAUNCH(true, false);
     constexpr int kStride =
         NetLayout<Lp, Hp>::size() + NetLayout<Lm, Hm>::size() + (PC1 > 0 ? Precond<(PC1 > 0 ? PC1 : 1), PC2>::size() : 0) + 1;
     hipLaunchKernelGGL((tile_apply_kernel<kStride>), dim3(1), dim3(1024), 0, st, partial, nblk, fo, params);
   } else if (mode == 1) {
-    DIPS_TILE_LAUNCH(true, 0);
+    DIPS_TILE_LAUNCH(true, false);
   } else {
-    DIPS_TILE_LAUNCH(false, 0);
+    DIPS_TILE_LAUNCH(false, false);
   }
 #undef DIPS_TILE_LAUNCH
 }
@@ -1084,7 +1081,7 @@ __global__ __launch_bounds__((TileCfg<Lm, Hm, Lp, Hp, PC1>::kThreads)) void tile
     TileStepArgs a = d.a;
     a.tile_begin = tb;
     a.ntiles = nt;
-    tile_step_body<Lm, Hm, Lp, Hp, true, 1, PC1, PC2, Act>(a, d.params, d.partial, k, nblk);
+    tile_step_body<Lm, Hm, Lp, Hp, true, PC1, PC2, Act>(a, d.params, d.partial, k, nblk);
   }
 }
 
