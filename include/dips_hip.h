@@ -267,8 +267,10 @@ int dips_batch_train(const dips_batch_problem_t* probs, int32_t nprob, int32_t n
 
 /* Shape of the batched steps (chosen by an autotuner, e.g. jax_dips.records.BatchEngine.autotune).
  * Each global step is one persistent launch of grid_blocks workgroups that take work items (problem p,
- * block k) from a device queue; problem p's step has min(blk_cap, its tile blocks) blocks, each writing
- * one partial row reduced in block order by the problem's optimizer workgroup.  blk_cap = 256 (or 0)
+ * block k) from a device queue; problem p's step has min(blk_cap, its tile blocks) blocks, each reduced
+ * to one partial row and these in block order by the problem's optimizer workgroup.  Blocks of many tiles are
+ * summed in four parts, which are work items of their own where that ends a step sooner; results do not depend
+ * on it, nor on grid_blocks.  blk_cap = 256 (or 0)
  * reproduces the single-problem step bit for bit; fewer blocks make larger work items. */
 typedef struct {
   int32_t blk_cap;      /* 1..256; 0: 256 */
@@ -293,8 +295,8 @@ int64_t dips_batch_workspace_cfg(const dips_batch_problem_t* probs, int32_t npro
 int dips_batch_setup(const dips_batch_problem_t* probs, int32_t nprob, int32_t nepochs, const dips_net_t* net,
                      const dips_opt_t* opt, const dips_batch_cfg_t* cfg, void* work, int64_t work_bytes,
                      dips_batch_plan_t* plan, void* stream);
-/* Enqueues nsteps global steps from the device step counter on (3 launches each: the persistent step,
- * the optimizer workgroups, the counter update); launches only, so a caller may capture them in a HIP
+/* Enqueues nsteps global steps from the device step counter on (2 launches each: the persistent step;
+ * the optimizer workgroups and the counter update); launches only, so a caller may capture them in a HIP
  * graph (e.g. one epoch, plan->max_steps / nepochs steps) and replay.  Steps past a problem's last
  * leave it unchanged. */
 int dips_batch_steps(const dips_net_t* net, const dips_batch_plan_t* plan, int32_t nsteps, void* work, void* stream);

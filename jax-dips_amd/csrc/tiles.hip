@@ -28,6 +28,7 @@
 #include <limits.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "dips_common.h"
@@ -39,6 +40,7 @@ namespace dips {
 
 constexpr int kTileCap = 64;                          // entries and rows of a packed tile
 constexpr int kMaxTileBlocks = 256;                   // one workgroup per CU
+constexpr int kSegs = 4;                              // parts of a block (batched steps, TileSeg)
 constexpr int kLdsStride = 68;                        // floats per staged operand row: 64 entries + 4
 constexpr int kStageFloats = 2 * 16 * kLdsStride;     // A and B operand stacks of one wavefront
 
@@ -99,7 +101,8 @@ __device__ __forceinline__ int64_t clamp64(int64_t v, int64_t lo, int64_t hi) { 
 typedef float row4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef const __attribute__((address_space(1))) row4 global_row4;
 
-// Reduce the partial rows (partial[b * kStride + p], b < nblk <= kMaxTileBlocks) in a fixed order, in float64,
+// Reduce the partial rows (partial[b * kStride + p], b < nblk <= kMaxTileBlocks; with nseg = kSegs those of a block's
+// parts first, in float32 as the step kernel adds them) in a fixed order, in float64,
 // and apply the optimizer to params / m / v; one workgroup.
 // A lane owns four neighbouring parameters (16-byte loads of a row) and a group of wavefronts every kGroups-th row;
 // the groups' sums meet in LDS and are added in order.  The kernel is a latency chain (rows -> norm ->
@@ -107,7 +110,7 @@ typedef const __attribute__((address_space(1))) row4 global_row4;
 // parameter was most of it: 20.7 -> 7.2 us (32 rows of 707), 11.7 -> 8.0 us (256 of 420), 6.3 -> 5.9 us (256 of 168).
 // kGroups depends on the shape only, so that every launch form adds in the same order.
 template <int kStride, int kTileWaves>
-__device__ void tile_reduce_apply(const float* partial, int nblk, const FusedOpt& fo, float* params) {
+__device__ void tile_reduce_apply(const float* partial, int nblk, int nseg, const FusedOpt& fo, float* params) {
   constexpr int kTileThreads = kTileWaves * DIPS_WAVE;
   constexpr int PT = kStride - 1;
   constexpr int kOwn = (PT + kTileThreads - 1) / kTileThreads;        // parameters updated per thread
@@ -138,19 +141,34 @@ __device__ void tile_reduce_apply(const float* partial, int nblk, const FusedOpt
   const int col = min(4 * (wave % kRowWaves * DIPS_WAVE + lane), kStride - 4);
   for (int g = wave / kRowWaves; g < kGroups && wave < kTeams * kRowWaves; g += kTeams) {
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    constexpr int kChunk = 16;  // rows in flight
-    for (int b0 = g; b0 < nblk; b0 += kChunk * kGroups) {
-      row4 v[kChunk];
+    // 16 rows in flight: of 16 blocks, or of 4 blocks in kSegs parts each
+    auto add = [&](auto segs) {
+      constexpr int kS = decltype(segs)::value, kChunk = 16 / kS;
+      for (int b0 = g; b0 < nblk; b0 += kChunk * kGroups) {
+        row4 v[kChunk][kS];
 #pragma unroll
-      for (int j = 0; j < kChunk; ++j)
-        v[j] = *(global_row4*)(partial + (int64_t)min(b0 + j * kGroups, nblk - 1) * kStride + col);
+        for (int j = 0; j < kChunk; ++j)
 #pragma unroll
-      for (int j = 0; j < kChunk; ++j)
-        if (b0 + j * kGroups < nblk) {
+          for (int k = 0; k < kS; ++k)
+            v[j][k] =
+                *(global_row4*)(partial + ((int64_t)min(b0 + j * kGroups, nblk - 1) * kS + k) * kStride + col);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[i] += (double)v[j][i];
-        }
-    }
+        for (int j = 0; j < kChunk; ++j)
+          if (b0 + j * kGroups < nblk) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              float t = v[j][0][i];
+#pragma unroll
+              for (int k = 1; k < kS; ++k) t += v[j][k][i];
+              acc[i] += (double)t;
+            }
+          }
+      }
+    };
+    if (nseg == 1)
+      add(std::integral_constant<int, 1>());
+    else
+      add(std::integral_constant<int, kSegs>());
 #pragma unroll
     for (int i = 0; i < 4; ++i) gsum[g][col + i] = acc[i];
   }
@@ -202,7 +220,7 @@ __device__ void tile_reduce_apply(const float* partial, int nblk, const FusedOpt
 template <int kStride>
 __global__ __launch_bounds__(1024) void tile_apply_kernel(const float* partial, int nblk, FusedOpt fo,
                                                          float* params) {
-  tile_reduce_apply<kStride, 16>(partial, nblk, fo, params);
+  tile_reduce_apply<kStride, 16>(partial, nblk, 1, fo, params);
 }
 
 typedef float f4 __attribute__((ext_vector_type(4)));
@@ -603,9 +621,16 @@ struct TileCfg {
 //
 // The body of one workgroup: block blk of nblk workgroups over the tiles of
 // a.  Writes the workgroup's partial row partial[blk * stride + p].
+// The part of a block's tiles that one call of the body takes: iterations [begin, end) of every wavefront (its tiles
+// are blk * waves + wave + i * nblk * waves), added to partial row `row` unless it is the row's first part.
+struct TileSeg {
+  int begin, end, row;
+  bool first;
+};
+
 template <int Lm, int Hm, int Lp, int Hp, bool kGrad, int PC1, int PC2, int Act>
-__device__ __forceinline__ void tile_step_body(const TileStepArgs& a, float* params, float* __restrict__ partial,
-                                               int blk, int nblk) {
+__device__ __forceinline__ void tile_step_body(const TileStepArgs& a, float* params, float* partial, int blk,
+                                               int nblk, const TileSeg& seg) {
   constexpr int kTileThreads = TileCfg<Lm, Hm, Lp, Hp, PC1>::kThreads;
   constexpr int kTileWaves = TileCfg<Lm, Hm, Lp, Hp, PC1>::kWaves;
   using NP = NetLayout<Lp, Hp>;
@@ -635,7 +660,8 @@ __device__ __forceinline__ void tile_step_body(const TileStepArgs& a, float* par
   float lsum = 0.0f;
 
   const int nw = nblk * kTileWaves;
-  const int t0 = blk * kTileWaves + wave;
+  const int t0 = blk * kTileWaves + wave + seg.begin * nw;
+  const int niter = seg.end - seg.begin;
   // slot data of the wavefront's next tile is loaded one tile ahead (the last
   // prefetch re-reads the final tile, unused)
   auto slot_of = [&](int t) { return (a.tile_begin + min(t, a.ntiles - 1)) * kTileCap + lane; };
@@ -646,7 +672,7 @@ __device__ __forceinline__ void tile_step_body(const TileStepArgs& a, float* par
   // marked here, by the wavefront's iteration index, for the second loop
   uint64_t longmask = 0;
   int iter = 0;
-  for (int t = t0; t < a.ntiles; t += nw, ++iter) {
+  for (int t = t0; t < a.ntiles && iter < niter; t += nw, ++iter) {
     // weights are re-read per tile (scalar loads that hit the scalar cache)
     // rather than held in vector registers across the loop
     const float* Praw = params;
@@ -724,7 +750,7 @@ __device__ __forceinline__ void tile_step_body(const TileStepArgs& a, float* par
   // its own so that its register demand does not add to the packed path's.
   iter = 0;
 #pragma unroll 1
-  for (int t = t0; t < a.ntiles; t += nw, ++iter) {
+  for (int t = t0; t < a.ntiles && iter < niter; t += nw, ++iter) {
     if (iter < 64 && !((longmask >> iter) & 1)) continue;  // a packed tile, done above
     const int64_t tb = a.tile_begin + t;
     const int64_t r0 = clamp64(gld(a.tile_row, tb), 0, a.nrows);
@@ -851,7 +877,8 @@ __device__ __forceinline__ void tile_step_body(const TileStepArgs& a, float* par
 #pragma unroll
       for (int w = 0; w < kTileWaves; ++w) s += red[w * stride + p];
     }
-    gst(partial, (int64_t)blk * stride + p, s);
+    const int64_t o = (int64_t)seg.row * stride + p;
+    gst(partial, o, seg.first ? s : gld(partial, o) + s);
   }
 }
 
@@ -867,7 +894,8 @@ __global__ __launch_bounds__((TileCfg<Lm, Hm, Lp, Hp, PC1>::kThreads)) void tile
   constexpr int kTileWaves = TileCfg<Lm, Hm, Lp, Hp, PC1>::kWaves;
   constexpr int stride = tile_stride<Lm, Hm, Lp, Hp, PC1, PC2>();
   const int nblk = (int)gridDim.x;
-  tile_step_body<Lm, Hm, Lp, Hp, kGrad, PC1, PC2, Act>(a, params, partial, (int)blockIdx.x, nblk);
+  tile_step_body<Lm, Hm, Lp, Hp, kGrad, PC1, PC2, Act>(a, params, partial, (int)blockIdx.x, nblk,
+                                                       TileSeg{0, INT_MAX, (int)blockIdx.x, true});
   if (!kFused) return;
 
   // One thread per workgroup fences and counts: the barrier completes the
@@ -884,7 +912,7 @@ __global__ __launch_bounds__((TileCfg<Lm, Hm, Lp, Hp, PC1>::kThreads)) void tile
   }
   __syncthreads();
   if (!am_last) return;
-  tile_reduce_apply<stride, kTileWaves>(partial, nblk, fo, params);
+  tile_reduce_apply<stride, kTileWaves>(partial, nblk, 1, fo, params);
 }
 
 // workgroups of a launch over ntiles tiles with waves wavefronts per workgroup
@@ -1013,32 +1041,41 @@ int tile_train_step(const dips_grid_t* g, const dips_records_t* rec, const dips_
 
 // ---------------------------------------------------------------------------
 // Batched training of many problems.  A global step is one persistent launch
-// whose workgroups pull items from a device work queue: item (p, k) is block k
+// whose workgroups take items: item (p, k) is block k
 // of the nblk_p workgroup blocks that problem p's step uses on its own
 // (nblk_p = min(cap, blocks for the tiles of its batch s mod nbatches_p)), and
 // writes exactly that block's partial row, whichever workgroup takes it.  Then
 // one reduction + optimizer workgroup per problem, in block order.  With
 // cap = kMaxTileBlocks every problem follows the trajectory the
-// single-problem two-launch step gives it, bit for bit.  The global step and
-// the queue head live in device memory (BatchCtrl), advanced by a one-thread
-// kernel after each step, so an epoch of launches can be captured in a graph
-// and replayed.
+// single-problem two-launch step gives it, bit for bit.
+// Items are the blocks of the problems that still run at this step, or, where that ends sooner, the kSegs parts of
+// each block (tile_segs, batch_items): a block's tiles are summed part by part in either case, so the result does not
+// depend on which it was, nor on the other problems.  12 problems of 2x16 networks, 32 blocks each (all of
+// a CU's matrix and vector issue for 120 us): with one problem left 32 of 256 CUs had work, with 12 the last third
+// of the blocks ran alone; 8.5 -> 5.7 ms for 28 steps.  The queue is asked when an item is done: asked
+// ahead, the items of a short last round go to the workgroups that were first, not to those that are free (+5%).
+// The global step and the queue head live in device memory, advanced by the apply launch's last
+// workgroup, so an epoch of launches can be captured in a graph and replayed.
 struct BatchDesc {
   TileStepArgs a;                   // tile_begin / ntiles are set per step
   const int64_t* batch_tile_begin;  // device copy, nbatches + 1
   int32_t nbatches;
   int32_t steps;
-  int32_t blk_begin;                // first item of the problem
-  int32_t blk_count;                // items of the problem: its most blocks over the batches
   float* params;
-  float* partial;                   // blk_count * stride floats
+  float* partial;                   // (most blocks, or blocks times parts, over the batches) * stride floats
   FusedOpt fo;
 };
 
+// followed by int32_t item_begin[nprob + 1]: the items of each problem at global step next
 struct BatchCtrl {
-  uint32_t queue;  // next item of the current global step
-  int32_t step;    // current global step
+  uint32_t queue;    // items taken beyond the first of each workgroup
+  int32_t step;      // the global step of the last step launch: read by the apply launch, written by the step launch
+  int32_t next;      // the global step of the next step launch: the other way round
+  int32_t split;     // whether the blocks' parts were items of their own in the last step launch (as step)
+  int32_t split_next;  // and are in the next (as next)
+  int32_t pad[3];
 };
+__device__ __forceinline__ int32_t* item_table(BatchCtrl* c) { return reinterpret_cast<int32_t*>(c + 1); }
 
 // the step's tile range and block count of problem d at global step s
 __device__ __forceinline__ bool batch_step_range(const BatchDesc& d, int s, int waves, int cap, int64_t& tb, int& nt,
@@ -1051,70 +1088,156 @@ __device__ __forceinline__ bool batch_step_range(const BatchDesc& d, int s, int 
   return true;
 }
 
+// Parts of a problem's blocks, a rule of its own sizes only: a block of many tiles is summed in kSegs parts (each from
+// zero, the parts added in order), so that one workgroup or kSegs of them may take it with the same result.  A part
+// costs about two tiles' time a wavefront (packing the weights, reducing over the workgroup): from 8 tiles a
+// wavefront on, and up to 64 blocks, beyond which a problem fills the device by itself.
+__host__ __device__ static inline int tile_segs(int64_t ntiles, int nblk, int waves, int& len) {
+  const int per_wave = (int)((ntiles + (int64_t)nblk * waves - 1) / ((int64_t)nblk * waves));
+  const int segs = nblk <= 64 && per_wave >= 8 ? kSegs : 1;
+  len = (per_wave + segs - 1) / segs;
+  return segs;
+}
+
+// a value and a problem's descriptor at wave-uniform addresses that the launch does not write: scalar loads into
+// scalar registers
+__device__ __forceinline__ int uld(const int32_t* p) { return *(const __attribute__((address_space(4))) int32_t*)p; }
+__device__ __forceinline__ BatchDesc uniform_desc(const BatchDesc* p) {
+  static_assert(sizeof(BatchDesc) % sizeof(uint64_t) == 0, "descriptor words");
+  constexpr int kWords = sizeof(BatchDesc) / sizeof(uint64_t);
+  const auto* const w = (const __attribute__((address_space(4))) uint64_t*)p;
+  uint64_t v[kWords];
+#pragma unroll
+  for (int i = 0; i < kWords; ++i) v[i] = w[i];
+  BatchDesc d;
+  __builtin_memcpy(&d, v, sizeof(d));
+  return d;
+}
+
 template <int Lm, int Hm, int Lp, int Hp, int PC1, int PC2, int Act>
 __global__ __launch_bounds__((TileCfg<Lm, Hm, Lp, Hp, PC1>::kThreads)) void tile_batch_step_kernel(
-    const BatchDesc* __restrict__ descs, int nprob, int nitems, int cap, BatchCtrl* __restrict__ ctrl) {
+    const BatchDesc* __restrict__ descs, int nprob, int cap, BatchCtrl* ctrl) {
   constexpr int kTileWaves = TileCfg<Lm, Hm, Lp, Hp, PC1>::kWaves;
-  const int s = ctrl->step;
+  const int s = uld(&ctrl->next), split = uld(&ctrl->split_next);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    ctrl->step = s;
+    ctrl->split = split;
+  }
+  const int32_t* const begin = item_table(ctrl);
+  const int nitems = uld(begin + nprob);
   __shared__ int item_s;
-  for (;;) {
-    __syncthreads();  // every thread has read the previous item
-    if (threadIdx.x == 0) item_s = (int)atomicAdd(&ctrl->queue, 1u);
-    __syncthreads();
-    const int item = item_s;
-    if (item >= nitems) return;
-    // owner problem: the last p with blk_begin <= item
+  int item = blockIdx.x;
+  while (item < nitems) {
+    // owner problem: the last p with begin[p] <= item (problems without items share their successor's begin)
     int lo = 0, hi = nprob - 1;
     while (lo < hi) {
       const int mid = (lo + hi + 1) >> 1;
-      if (descs[mid].blk_begin <= item)
+      if (uld(begin + mid) <= item)
         lo = mid;
       else
         hi = mid - 1;
     }
-    const BatchDesc& d = descs[lo];
+    const BatchDesc d = uniform_desc(descs + lo);
     int64_t tb;
-    int nt, nblk;
-    if (!batch_step_range(d, s, kTileWaves, cap, tb, nt, nblk)) continue;
-    const int k = item - d.blk_begin;
-    if (k >= nblk) continue;
+    int nt, nblk, len;
+    if (!batch_step_range(d, s, kTileWaves, cap, tb, nt, nblk)) return;  // not reached: a problem with items runs
+    const int segs = tile_segs(nt, nblk, kTileWaves, len);
+    const int k = item - uld(begin + lo);
     TileStepArgs a = d.a;
     a.tile_begin = tb;
     a.ntiles = nt;
-    tile_step_body<Lm, Hm, Lp, Hp, true, PC1, PC2, Act>(a, d.params, d.partial, k, nblk);
+    const int parts = split ? segs : 1;  // items of a block
+    for (int q = 0; q < segs / parts; ++q) {
+      const int part = k % parts + q;
+      tile_step_body<Lm, Hm, Lp, Hp, true, PC1, PC2, Act>(a, d.params, d.partial, k / parts, nblk,
+                                                           TileSeg{part * len, part * len + len, k, q == 0});
+      __syncthreads();  // the body's LDS is free; every thread has read the previous item_s
+    }
+    if (threadIdx.x == 0) item_s = (int)(gridDim.x + atomicAdd(&ctrl->queue, 1u));
+    __syncthreads();
+    item = __builtin_amdgcn_readfirstlane(item_s);
   }
 }
 
+// items of every problem at global step s, for a launch of about grid workgroups, and the empty queue; one wavefront
+__device__ void batch_items(const BatchDesc* descs, int nprob, int waves, int cap, int grid, int s, BatchCtrl* ctrl) {
+  const int lane = threadIdx.x;
+  int32_t* const begin = item_table(ctrl);
+  auto items = [&](int p, int& segs, int& len) {
+    int64_t tb;
+    int nt, nblk;
+    segs = 1;
+    len = 0;
+    if (p >= nprob || !batch_step_range(descs[p], s, waves, cap, tb, nt, nblk)) return 0;
+    segs = tile_segs(nt, nblk, waves, len);
+    return nblk;
+  };
+  // whole blocks or their parts as items: rounds of the grid times an item's length (in tiles a wavefront, the fixed
+  // cost of an item counted as 2)
+  auto wave_max = [](int v) {
+    for (int o = 1; o < DIPS_WAVE; o *= 2) v = max(v, __shfl_xor(v, o, DIPS_WAVE));
+    return v;
+  };
+  int64_t whole = 0, parts = 0;
+  int whole_len = 0, part_len = 0;
+  for (int p0 = 0; p0 < nprob; p0 += DIPS_WAVE) {
+    int segs, len;
+    const int nblk = items(p0 + lane, segs, len);
+    whole += dips_wave_sum_i(nblk);
+    parts += dips_wave_sum_i(nblk * segs);
+    whole_len = max(whole_len, wave_max(len * segs));
+    part_len = max(part_len, wave_max(len));
+  }
+  const bool split = parts < INT_MAX && (parts + grid - 1) / grid * (part_len + 2) <
+                                            (whole + grid - 1) / grid * (whole_len + 2);
+  int base = 0;
+  for (int p0 = 0; p0 < nprob; p0 += DIPS_WAVE) {
+    int segs, len;
+    const int nblk = items(p0 + lane, segs, len);
+    const int mine = split ? nblk * segs : nblk;
+    int sum = mine;  // inclusive scan
+    for (int o = 1; o < DIPS_WAVE; o *= 2) {
+      const int t = __shfl_up(sum, o, DIPS_WAVE);
+      if (lane >= o) sum += t;
+    }
+    if (p0 + lane < nprob) gst(begin, p0 + lane, base + sum - mine);
+    base += __shfl(sum, DIPS_WAVE - 1, DIPS_WAVE);
+  }
+  if (lane == 0) {
+    gst(begin, nprob, base);
+    ctrl->queue = 0u;
+    ctrl->next = s;
+    ctrl->split_next = split ? 1 : 0;
+  }
+}
+
+// workgroup p < nprob: problem p's reduction and optimizer; the last one prepares the next global step
 template <int kStride, int kWaves>
-__global__ __launch_bounds__(1024) void tile_batch_apply_kernel(const BatchDesc* __restrict__ descs, int cap,
-                                                                const BatchCtrl* __restrict__ ctrl) {
+__global__ __launch_bounds__(1024) void tile_batch_apply_kernel(const BatchDesc* __restrict__ descs, int nprob,
+                                                                int cap, int grid, BatchCtrl* ctrl) {
+  const int s = ctrl->step, split = ctrl->split;
+  if ((int)blockIdx.x == nprob) {
+    if (threadIdx.x < DIPS_WAVE) batch_items(descs, nprob, kWaves, cap, grid, s + 1, ctrl);
+    return;
+  }
   const BatchDesc& d = descs[blockIdx.x];
   int64_t tb;
   int nt, nblk;
-  if (!batch_step_range(d, ctrl->step, kWaves, cap, tb, nt, nblk)) return;
-  tile_reduce_apply<kStride, 16>(d.partial, nblk, d.fo, d.params);
+  if (!batch_step_range(d, s, kWaves, cap, tb, nt, nblk)) return;
+  int len;
+  tile_reduce_apply<kStride, 16>(d.partial, nblk, split ? tile_segs(nt, nblk, kWaves, len) : 1, d.fo, d.params);
 }
 
-// after a step: empty queue, next global step
-__global__ void batch_ctrl_next_kernel(BatchCtrl* ctrl) {
-  if (threadIdx.x == 0) {
-    ctrl->queue = 0u;
-    ctrl->step = ctrl->step + 1;
-  }
-}
-
-__global__ void batch_ctrl_init_kernel(BatchCtrl* ctrl, int step) {
-  if (threadIdx.x == 0) {
-    ctrl->queue = 0u;
-    ctrl->step = step;
-  }
+__global__ void batch_ctrl_init_kernel(const BatchDesc* descs, int nprob, int waves, int cap, int grid,
+                                       BatchCtrl* ctrl) {
+  batch_items(descs, nprob, waves, cap, grid, 0, ctrl);
 }
 
 namespace {
 struct BatchLayout {
   int64_t desc_off, table_off, partial_off, ctrl_off, bytes;
   int32_t nblk_total;
-  std::vector<int32_t> blk_count;
+  std::vector<int32_t> rows;  // partial rows of each problem
 };
 
 constexpr int64_t kAlign = 256;
@@ -1145,26 +1268,29 @@ int batch_layout(const dips_batch_problem_t* probs, int32_t nprob, const dips_ne
   }
   const int64_t stride = partial_stride(net);
   int64_t tables = 0, partials = 0, blocks = 0;
-  L.blk_count.assign(nprob, 0);
+  L.rows.assign(nprob, 0);
   for (int p = 0; p < nprob; ++p) {
     const dips_batch_problem_t& q = probs[p];
     if (!q.batch_tile_begin || q.nbatches < 1 || q.batch_size < 1) {
       set_error("batch train: problem " + std::to_string(p) + ": invalid batch table");
       return DIPS_EINVAL;
     }
-    int cnt = 1;
+    int cnt = 1, rows = 1;
     for (int b = 0; b < q.nbatches; ++b) {
       const int64_t nt = q.batch_tile_begin[b + 1] - q.batch_tile_begin[b] - 1;
       if (nt < 1 || q.batch_tile_begin[b] < 0 || q.batch_tile_begin[b + 1] > q.tiles.nbounds) {
         set_error("batch train: problem " + std::to_string(p) + ": batch without tiles or outside the tile table");
         return DIPS_EINVAL;
       }
-      cnt = std::max(cnt, std::min(tile_blocks(nt, waves), cap));
+      const int nblk = std::min(tile_blocks(nt, waves), cap);
+      int len;
+      cnt = std::max(cnt, nblk);
+      rows = std::max(rows, nblk * tile_segs(nt, nblk, waves, len));
     }
-    L.blk_count[p] = cnt;
+    L.rows[p] = rows;
     blocks += cnt;
     tables += q.nbatches + 1;
-    partials += (int64_t)cnt * stride;
+    partials += (int64_t)rows * stride;
   }
   if (blocks > INT_MAX / 2) {
     set_error("batch train: too many workgroups");
@@ -1175,7 +1301,7 @@ int batch_layout(const dips_batch_problem_t* probs, int32_t nprob, const dips_ne
   L.table_off = align_up((int64_t)sizeof(BatchDesc) * nprob);
   L.partial_off = align_up(L.table_off + (int64_t)sizeof(int64_t) * tables);
   L.ctrl_off = align_up(L.partial_off + (int64_t)sizeof(float) * partials);
-  L.bytes = align_up(L.ctrl_off + (int64_t)sizeof(BatchCtrl));
+  L.bytes = align_up(L.ctrl_off + (int64_t)sizeof(BatchCtrl) + (int64_t)sizeof(int32_t) * (nprob + 1));
   return DIPS_OK;
 }
 
@@ -1205,12 +1331,11 @@ static void batch_launch_shape(const BatchDesc* descs, BatchCtrl* ctrl, const di
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
   (void)lds_set;
   hipLaunchKernelGGL((tile_batch_step_kernel<Lm, Hm, Lp, Hp, PC1, PC2, Act>), dim3(plan.grid_blocks),
-                     dim3(TileCfg<Lm, Hm, Lp, Hp, PC1>::kThreads), lds, st, descs, plan.nprob, plan.nitems,
-                     plan.blk_cap, ctrl);
+                     dim3(TileCfg<Lm, Hm, Lp, Hp, PC1>::kThreads), lds, st, descs, plan.nprob, plan.blk_cap,
+                     ctrl);
   constexpr int kStride = tile_stride<Lm, Hm, Lp, Hp, PC1, PC2>();
-  hipLaunchKernelGGL((tile_batch_apply_kernel<kStride, kWaves>), dim3(plan.nprob), dim3(1024), 0, st, descs,
-                     plan.blk_cap, ctrl);
-  hipLaunchKernelGGL(batch_ctrl_next_kernel, dim3(1), dim3(64), 0, st, ctrl);
+  hipLaunchKernelGGL((tile_batch_apply_kernel<kStride, kWaves>), dim3(plan.nprob + 1), dim3(1024), 0, st, descs,
+                     plan.nprob, plan.blk_cap, plan.grid_blocks, ctrl);
 }
 
 int batch_setup(const dips_batch_problem_t* probs, int32_t nprob, int32_t nepochs, const dips_net_t* net,
@@ -1232,7 +1357,6 @@ int batch_setup(const dips_batch_problem_t* probs, int32_t nprob, int32_t nepoch
   char* base = static_cast<char*>(work);
   std::vector<BatchDesc> descs(nprob);
   std::vector<int64_t> tables;
-  int32_t blk = 0;
   int64_t maxsteps = 0;
   int64_t poff = 0;
   const int64_t stride = partial_stride(net);
@@ -1264,12 +1388,9 @@ int batch_setup(const dips_batch_problem_t* probs, int32_t nprob, int32_t nepoch
     tables.insert(tables.end(), q.batch_tile_begin, q.batch_tile_begin + q.nbatches + 1);
     d.nbatches = q.nbatches;
     d.steps = (int32_t)steps;
-    d.blk_begin = blk;
-    d.blk_count = L.blk_count[p];
-    blk += L.blk_count[p];
     d.params = q.params;
     d.partial = reinterpret_cast<float*>(base + L.partial_off) + poff;
-    poff += (int64_t)L.blk_count[p] * stride;
+    poff += (int64_t)L.rows[p] * stride;
     d.fo = FusedOpt{*opt, 1.0f / (float)q.batch_size, q.m, q.v, q.count, q.loss_hist, q.loss_cap, nullptr};
   }
   int grid = 0;
@@ -1288,8 +1409,9 @@ int batch_setup(const dips_batch_problem_t* probs, int32_t nprob, int32_t nepoch
     e = hipMemcpyAsync(base + L.table_off, tables.data(), sizeof(int64_t) * tables.size(), hipMemcpyHostToDevice,
                        stream);
   if (e == hipSuccess) {
-    hipLaunchKernelGGL(batch_ctrl_init_kernel, dim3(1), dim3(64), 0, stream,
-                       reinterpret_cast<BatchCtrl*>(base + L.ctrl_off), 0);
+    hipLaunchKernelGGL(batch_ctrl_init_kernel, dim3(1), dim3(DIPS_WAVE), 0, stream,
+                       reinterpret_cast<const BatchDesc*>(base + L.desc_off), nprob, tile_waves_of(net), cap, grid,
+                       reinterpret_cast<BatchCtrl*>(base + L.ctrl_off));
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipStreamSynchronize(stream);
