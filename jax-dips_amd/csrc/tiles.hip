@@ -599,16 +599,277 @@ struct PrecondGrad {
   }
 };
 
+// ---- phase networks as chains of 16x16x4 products
+// A tile's 64 slots are four sub-tiles of 16; lane 16 g + p holds features 4 g .. 4 g + 3 of slot 16 s + p of
+// every sub-tile s (16 registers per hidden layer, widths below 16 padded with zero weights).  That is the
+// accumulator layout of v_mfma_f32_16x16x4f32 and, with the contraction index in the order k = 4 g + r, also its B
+// operand, so the hidden layers chain without data movement and the weights are 4 registers per lane and
+// layer, read from a copy in LDS, instead of a scalar operand per multiply-add.
+// Outputs return to one lane per slot and seeds leave it with three lane-row swaps each.
+// Bound by issue, two wavefronts per SIMD: 68 matrix instructions (32 cycles each, beside which the vector unit idles),
+// 64 exp / rcp and about 250 other vector instructions a tile, 4.8K cycles measured; evaluated per lane, with a scalar
+// operand per multiply-add, 1.7K vector instructions.  12-problem sweep of 2x16 networks: 5.78 -> 4.78 ms.
+
+// weights of one network, packed per lane (floats): layer 0 [64]; per further hidden layer W [64][4], its transpose
+// [64][4], bias [16]; Wout [16], bout
+template <int L, int H, int Act>
+struct ChainNet {
+  static constexpr int layer(int l) { return 64 + (l - 1) * 528; }
+  static constexpr int wt(int l) { return layer(l) + 256; }
+  static constexpr int bias(int l) { return layer(l) + 512; }
+  static constexpr int wout() { return layer(L); }
+  static constexpr int size() { return wout() + 20; }
+  // tanh networks: the forward weights carry the factor of dips_tanh_exp2's argument
+  static constexpr float kScale = Act == kActTanh ? kTanhExp2Scale : 1.0f;
+
+  __device__ static void pack(const float* P, float* W, int nthreads) {
+    using NL = NetLayout<L, H>;
+    for (int i = threadIdx.x; i < size(); i += nthreads) {
+      int src = -1;  // parameter index
+      float scale = kScale;
+      if (i < 64) {
+        const int g = i >> 4, o = i & 15;
+        if (o < H) src = g < 3 ? NL::w(0) + g * H + o : NL::b(0) + o;
+      } else if (i < wout()) {
+        const int l = 1 + (i - 64) / 528, q = (i - 64) % 528, ln = (q & 255) >> 2, r = q & 3;
+        const int f = 4 * (ln >> 4) + r, m = ln & 15;  // k = 4 g + r and the lane's row
+        const int wl = NL::w(1) + (l - 1) * (H * H + H);
+        if (q < 512) {
+          const int from = q < 256 ? f : m, to = q < 256 ? m : f;
+          if (from < H && to < H) src = wl + from * H + to;
+          if (q >= 256) scale = 1.0f;
+        } else if (q - 512 < H) {
+          src = wl + H * H + q - 512;
+        }
+      } else {
+        const int q = i - wout();
+        src = q < H ? NL::wout() + q : q == 16 ? NL::bout() : -1;
+        scale = 1.0f;
+      }
+      const float v = gld(P, src < 0 ? 0 : src);
+      W[i] = src < 0 ? 0.0f : scale * v;
+    }
+  }
+};
+
+__device__ __forceinline__ void swap32(float& a, float& b) {
+  const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(v[0]);
+  b = __uint_as_float(v[1]);
+}
+__device__ __forceinline__ void swap16(float& a, float& b) {
+  const auto v = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(v[0]);
+  b = __uint_as_float(v[1]);
+}
+// lane 16 s + p receives the sum over g of v[s] of lane 16 g + p
+__device__ __forceinline__ float gather_slots(float (&v)[4]) {
+  swap32(v[0], v[2]);  // rows 0, 1 / 2, 3 of the sum: sub-tile 0 / 2
+  swap32(v[1], v[3]);
+  float a = v[0] + v[2], b = v[1] + v[3];
+  swap16(a, b);
+  return a + b;
+}
+// v[s] = x of lane 16 s + p
+__device__ __forceinline__ void spread_slots(float x, float (&v)[4]) {
+  v[0] = v[1] = x;
+  swap16(v[0], v[1]);  // rows 0 0 2 2 / 1 1 3 3
+  v[2] = v[0];
+  v[3] = v[1];
+  swap32(v[0], v[2]);
+  swap32(v[1], v[3]);
+}
+
+template <int Act>
+__device__ __forceinline__ float chain_act(float c) {
+  return Act == kActTanh ? dips_tanh_exp2(c) : act_f<Act>(c);
+}
+
+// u of this lane's slot; xin[s] = coordinate g (1 for g = 3) of slot 16 s + p; act[l][4 s + r]
+template <int L, int H, int Act, int LA>
+__device__ __forceinline__ float chain_forward(const float* W, int lane, const float (&xin)[4], float (&act)[LA][16]) {
+  using CN = ChainNet<L, H, Act>;
+  const float w0 = W[lane];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const f4 c = __builtin_amdgcn_mfma_f32_16x16x4f32(w0, xin[s], f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) act[0][4 * s + r] = chain_act<Act>(c[r]);
+  }
+#pragma unroll
+  for (int l = 1; l < L; ++l) {
+    const f4 w = *reinterpret_cast<const f4*>(W + CN::layer(l) + 4 * lane);
+    const f4 b = *reinterpret_cast<const f4*>(W + CN::bias(l) + 4 * (lane >> 4));
+    f4 c[4] = {b, b, b, b};
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        c[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[r], act[l - 1][4 * s + r], c[s], 0, 0, 0);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) act[l][4 * s + r] = chain_act<Act>(c[s][r]);
+  }
+  const f4 wo = *reinterpret_cast<const f4*>(W + CN::wout() + 4 * (lane >> 4));
+  float v[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    v[s] = act[L - 1][4 * s] * wo[0];
+#pragma unroll
+    for (int r = 1; r < 4; ++r) v[s] = fmaf(act[L - 1][4 * s + r], wo[r], v[s]);
+  }
+  return gather_slots(v) + W[CN::wout() + 16];
+}
+
+// gradient accumulators of one network
+template <int L, int H, bool kGrad>
+struct ChainGrad {
+  f4 w[kGrad ? L : 1];                   // block 0: rows x, y, z, 1; block l: rows of a_{l-1}; columns of delta_l
+  float b[kGrad && L > 1 ? L - 1 : 1][4];  // per-lane partial sums of the biases of layers 1 ..
+  float wo[4];
+  float bo;
+
+  __device__ __forceinline__ void zero() {
+#pragma unroll
+    for (int l = 0; l < (kGrad ? L : 1); ++l) w[l] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int l = 0; l < (kGrad && L > 1 ? L - 1 : 1); ++l)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) b[l][r] = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) wo[r] = 0.0f;
+    bo = 0.0f;
+  }
+
+  __device__ __forceinline__ void swap(ChainGrad& o) {
+    auto sw = [](auto& x, auto& y) {
+      const auto t = x;
+      x = y;
+      y = t;
+    };
+    sw(bo, o.bo);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sw(wo[r], o.wo[r]);
+#pragma unroll
+    for (int l = 0; l < (kGrad ? L : 1); ++l) sw(w[l], o.w[l]);
+#pragma unroll
+    for (int l = 0; l < (kGrad && L > 1 ? L - 1 : 1); ++l)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sw(b[l][r], o.b[l][r]);
+  }
+
+  // one tile (chunk) of slots: seed of this lane's slot (0 for the slots of the other network), activations of
+  // chain_forward; wave-uniform call
+  template <int Act, int LA>
+  __device__ __forceinline__ void add(const float* W, float* AT, float* BT, int lane, const float (&xin)[4], float seed,
+                                      const float (&act)[LA][16]) {
+    using CN = ChainNet<L, H, Act>;
+    const int g = lane >> 4, p = lane & 15;
+    float sd[4], d[16];
+    spread_slots(seed, sd);
+    const f4 wout = *reinterpret_cast<const f4*>(W + CN::wout() + 4 * g);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float a = act[L - 1][4 * s + r];
+        wo[r] = fmaf(sd[s], a, wo[r]);
+        d[4 * s + r] = sd[s] * wout[r] * act_grad<Act>(a);
+      }
+    bo += seed;
+#pragma unroll
+    for (int l = L - 1; l >= 0; --l) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (l > 0) AT[(4 * g + r) * kLdsStride + 16 * s + p] = act[l > 0 ? l - 1 : 0][4 * s + r];
+          BT[(4 * g + r) * kLdsStride + 16 * s + p] = d[4 * s + r];
+        }
+        if (l == 0) AT[g * kLdsStride + 16 * s + p] = xin[s];
+      }
+      __builtin_amdgcn_wave_barrier();
+      if (l > 0) {
+        const f4 wt = *reinterpret_cast<const f4*>(W + CN::wt(l) + 4 * lane);
+        f4 c[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) c[s] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int s = 0; s < 4; ++s) c[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(wt[r], d[4 * s + r], c[s], 0, 0, 0);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            b[l - 1][r] += d[4 * s + r];
+            d[4 * s + r] = c[s][r] * act_grad<Act>(act[l - 1][4 * s + r]);
+          }
+      }
+      stage_mfma(AT, BT, lane, w[l]);
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+
+  // this wavefront's sums into red[off .. off + NetLayout::size())
+  __device__ __forceinline__ void flush(float* red, int off, int lane) {
+    if constexpr (kGrad) {
+      using NL = NetLayout<L, H>;
+#pragma unroll
+      for (int blk = 0; blk < L; ++blk)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = 4 * (lane >> 4) + r, j = lane & 15;
+          int q = -1;
+          if (j < H) {
+            if (blk == 0)
+              q = i < 3 ? NL::w(0) + i * H + j : i == 3 ? NL::b(0) + j : -1;
+            else if (i < H)
+              q = NL::w(blk) + i * H + j;
+          }
+          if (q >= 0) red[off + q] = w[blk][r];
+        }
+      auto row_sum = [](float v) {
+        v += dips_dpp_f<0x111, 0xF, true>(v);
+        v += dips_dpp_f<0x112, 0xF, true>(v);
+        v += dips_dpp_f<0x114, 0xF, true>(v);
+        v += dips_dpp_f<0x118, 0xF, true>(v);
+        return v;  // lane 15 of each row of 16: the row's sum
+      };
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int f = 4 * (lane >> 4) + r;
+        const bool mine = (lane & 15) == 15 && f < H;
+        const float v = row_sum(wo[r]);
+        if (mine) red[off + NL::wout() + f] = v;
+#pragma unroll
+        for (int l = 1; l < L; ++l) {
+          const float t = row_sum(b[l - 1][r]);
+          if (mine) red[off + NL::b(l) + f] = t;
+        }
+      }
+      const float v = dips_wave_sum(bo);
+      if (lane == 0) red[off + NL::bout()] = v;
+    }
+  }
+};
+
 // Workgroup size per shape: 16 wavefronts (four per SIMD, 128 registers each)
 // unless both networks have two or more hidden layers on the matrix cores,
 // which need more registers per lane: then 8 wavefronts.
+// The chain form serves networks of one shape with two or more layers of width 13..16.  Narrower networks would be
+// padded to 16 (128^3 sphere with a 2x10 network 0.76 -> 0.97 ms an epoch), one layer has nothing to chain
+// (32^3 LPBE, 1x16: 42.2 -> 43.7 us).
 template <int Lm, int Hm, int Lp, int Hp, int PC1 = 0>
 struct TileCfg {
+  static constexpr bool kChain = Lm >= 2 && Lp == Lm && Hp == Hm && MfmaGradWide<Hm>::value && PC1 == 0;
   static constexpr bool kWide = (Lm >= 2 && Lp >= 2 && MfmaGrad<Hm>::value && MfmaGrad<Hp>::value) || PC1 > 0 ||
                                 MfmaGradWide<Hm>::value || MfmaGradWide<Hp>::value;
   static constexpr int kThreads = kWide ? 512 : 1024;
   static constexpr int kWaves = kThreads / DIPS_WAVE;
-  static constexpr size_t kLdsBytes = sizeof(float) * kStageFloats * kWaves;
+  static constexpr int kNet = kStageFloats * kWaves;  // chain form: the packed networks
+  static constexpr size_t kLdsBytes = sizeof(float) * (kNet + (kChain ? 2 * ChainNet<Lm, Hm, 0>::size() : 0));
 };
 
 // kFused: the last workgroup also reduces the partial rows and applies the optimizer.
@@ -628,9 +889,216 @@ struct TileSeg {
   bool first;
 };
 
+// The chain form of the body (below: the per-lane form, same arguments); both networks have the same shape.  The
+// phases of a tile go through one copy of the code: the phase's weights are an LDS offset, its accumulators are
+// swapped with the other phase's when the phase changes.
+template <int L, int H, bool kGrad, int Act>
+__device__ __forceinline__ void tile_chain_body(const TileStepArgs& a, const float* params, float* partial, int blk,
+                                                int nblk, const TileSeg& seg) {
+  using Cfg = TileCfg<L, H, L, H>;
+  using CN = ChainNet<L, H, Act>;
+  constexpr int PP = NetLayout<L, H>::size();
+  constexpr int PT = 2 * PP;
+  extern __shared__ f4 tile_lds[];
+  float* const lds = reinterpret_cast<float*>(tile_lds);
+  const int lane = threadIdx.x & (DIPS_WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / DIPS_WAVE);
+  float* const AT = lds + wave * kStageFloats;
+  float* const BT = AT + 16 * kLdsStride;
+  float* const W = lds + Cfg::kNet;  // + network, - network
+  if (seg.first) {
+    CN::pack(params, W, Cfg::kThreads);
+    CN::pack(params + PP, W + CN::size(), Cfg::kThreads);
+  }
+
+  ChainGrad<L, H, kGrad> gc, go;  // of the phase at work (0: +, 1: -) and of the other
+  gc.zero();
+  go.zero();
+  float lsum = 0.0f;
+  const int g = lane >> 4, p = lane & 15;
+
+  const int nw = nblk * Cfg::kWaves;
+  const int t0 = blk * Cfg::kWaves + wave + seg.begin * nw;
+  const int niter = t0 < a.ntiles ? min((a.ntiles - t0 + nw - 1) / nw, seg.end - seg.begin) : 0;
+  const float *const csx = a.sx, *const csy = a.sy, *const csz = a.sz;
+  const float* const coord = g == 0 ? csx : g == 1 ? csy : csz;
+  __syncthreads();  // the packed weights
+  uint64_t longmask = 0;  // as in the per-lane form
+  // 64 tiles of the wavefront at a time: which hold slots of which phase, then the + tiles, then the - tiles
+#pragma unroll 1
+  for (int i0 = 0; i0 < niter; i0 += 64) {
+    const int cnt = min(64, niter - i0);
+    auto slot_of = [&](int it) { return (a.tile_begin + t0 + (int64_t)(i0 + it) * nw) * kTileCap; };
+    uint64_t mask[2] = {0, 0};
+#pragma unroll 4
+    for (int it = 0; it < cnt; ++it) {
+      const uint32_t info = gld(a.sinfo, slot_of(it) + lane);
+      const bool on = (info & kSlotUsed) != 0, plus = (info & kSlotPlus) != 0;
+      if (__any(on && plus)) mask[0] |= 1ull << it;
+      if (__any(on && !plus)) mask[1] |= 1ull << it;
+    }
+    if (i0 == 0) longmask = ~(mask[0] | mask[1]);
+#pragma unroll 1
+    for (int ph = 0; ph < 2; ++ph) {
+      const float* const Wc = W + ph * CN::size();
+      uint64_t todo = ph == 0 ? mask[0] : mask[1];
+      const uint64_t both = mask[0] & mask[1];
+      // slot data of the next tile is loaded one tile ahead (the last prefetch re-reads the final tile, unused):
+      // info, weight and constant of this lane's slot, coordinate g of the four slots 16 s + p
+      uint32_t n_info = 0;
+      float n_w = 0.0f, n_c = 0.0f, n_x[4] = {};
+      auto load = [&](int it) {
+        const int64_t s0 = slot_of(it);
+        n_info = gld(a.sinfo, s0 + lane);
+        n_w = gld(a.sw, s0 + lane);
+        n_c = gld(a.sc, s0 + lane);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) n_x[s] = gld(coord, s0 + 16 * s + p);
+      };
+      int it = todo ? __builtin_ctzll(todo) : 0;
+      if (todo) load(it);
+#pragma unroll 1
+      while (todo) {
+        todo &= todo - 1;
+        const bool mixed = (both >> it) & 1;
+        if (todo) it = __builtin_ctzll(todo);
+        const uint32_t info = n_info;
+        const float w = n_w, c = n_c;
+        float xin[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) xin[s] = g == 3 ? 1.0f : n_x[s];
+        load(it);
+        const bool on = (info & kSlotUsed) != 0;
+        const int phase = (info & kSlotPlus) != 0 ? 0 : 1;
+        const int head = on ? (int)(info & 63u) : lane;
+        const int last = on ? (int)((info >> 6) & 63u) : lane;
+        // a tile of both phases: the other network's values too (its turn comes in the other loop)
+        float u = 0.0f;
+        float act[L][16];
+#pragma unroll 1
+        for (int q = mixed ? 0 : 1; q < 2; ++q) {
+          const int net = q ? ph : 1 - ph;
+          const float v0 = chain_forward<L, H, Act>(W + net * CN::size(), lane, xin, act);
+          u = phase == net ? v0 : u;
+        }
+        float v = on ? fmaf(w, u, c) : 0.0f;  // c is nonzero only in the row's last slot
+        // segmented inclusive scan: lane l ends with the sum of lanes head(l)..l
+        v = dips_segmented_scan(v, lane, head);
+        const float r = __shfl(v, last, DIPS_WAVE);
+        if (on && lane == last && !(mixed && ph == 1)) lsum = fmaf(0.5f * r, r, lsum);
+        if constexpr (kGrad)
+          gc.template add<Act>(Wc, AT, BT, lane, xin, on && phase == ph ? r * w : 0.0f, act);
+      }
+      gc.swap(go);
+    }
+  }
+  // long rows (tiles skipped above): one wavefront per row, 64 entries per
+  // chunk; the gradient pass recomputes the forward activations
+  int cur = 0;  // gc's phase
+  int iter = 0;
+#pragma unroll 1
+  for (int t = t0; iter < niter; t += nw, ++iter) {
+    if (iter < 64 && !((longmask >> iter) & 1)) continue;  // a packed tile, done above
+    const int64_t tb = a.tile_begin + t;
+    const int64_t r0 = clamp64(gld(a.tile_row, tb), 0, a.nrows);
+    const int64_t r1 = clamp64(gld(a.tile_row, tb + 1), r0, a.nrows);
+    // the tiles without slots: more than 64 rows or slots (tile_slots_kernel)
+    if (r1 - r0 <= kTileCap) {
+      int len = 0;
+      if (lane < r1 - r0) len = max(gld(a.row_ptr, r0 + lane + 1) - gld(a.row_ptr, r0 + lane), 1);
+      if (dips_wave_sum_i(len) <= kTileCap) continue;
+    }
+#pragma unroll 1
+    for (int64_t row = r0; row < r1; ++row) {
+      const int pt = gld(a.row_point, row);
+      float px, py, pz;
+      if (!point_xyz(a.ps, pt, px, py, pz)) continue;
+      const int64_t beg = clamp64(gld(a.row_ptr, row), 0, a.nnz);
+      const int64_t end = clamp64(gld(a.row_ptr, row + 1), beg, a.nnz);
+      // pass 0: the row's sum over both phases; passes 1, 2: the gradient of the -, + network
+      float acc = 0.0f, r = 0.0f;
+#pragma unroll 1
+      for (int pass = 0; pass < (kGrad ? 3 : 1); ++pass) {
+#pragma unroll 1
+        for (int64_t base = beg; base < end; base += DIPS_WAVE) {
+          const int64_t e = base + lane;
+          const bool on = e < end;
+          float x = 0.0f, y = 0.0f, z = 0.0f, we = 0.0f;
+          int phase = 1;
+          if (on) {
+            const uint32_t code = gld(a.ent_code, e);
+            int ox, oy, oz;
+            dips_decode_offset(code, ox, oy, oz);
+            x = px + (float)ox * a.hx;
+            y = py + (float)oy * a.hy;
+            z = pz + (float)oz * a.hz;
+            we = gld(a.ent_w, e);
+            phase = (code & 128u) != 0 ? 0 : 1;
+          }
+          float xin[4];
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            const float vx = __shfl(x, 16 * s + p, DIPS_WAVE), vy = __shfl(y, 16 * s + p, DIPS_WAVE),
+                        vz = __shfl(z, 16 * s + p, DIPS_WAVE);
+            xin[s] = g == 0 ? vx : g == 1 ? vy : g == 2 ? vz : 1.0f;
+          }
+          float u = 0.0f;
+#pragma unroll 1
+          for (int ph = pass == 1 ? 1 : 0; ph < (pass == 2 ? 1 : 2); ++ph) {
+            if (!__any(on && phase == ph)) continue;
+            const float* const Wc = W + ph * CN::size();
+            float act[L][16];
+            const float v0 = chain_forward<L, H, Act>(Wc, lane, xin, act);
+            u = phase == ph ? v0 : u;
+            if (kGrad && pass > 0) {
+              if (ph != cur) {
+                gc.swap(go);
+                cur = ph;
+              }
+              gc.template add<Act>(Wc, AT, BT, lane, xin, phase == ph ? r * we : 0.0f, act);
+            }
+          }
+          if (pass == 0) acc = on ? fmaf(we, u, acc) : acc;
+        }
+        if (pass == 0) {
+          r = dips_wave_sum(acc) + gld(a.row_c, row);
+          if (lane == 0) lsum = fmaf(0.5f * r, r, lsum);
+        }
+      }
+    }
+  }
+  if (cur == 1) gc.swap(go);
+
+  // workgroup reduction: per-wavefront sums into LDS (the staging area is
+  // reused), then the wavefronts are added in order
+  constexpr int stride = PT + 1;
+  __syncthreads();
+  float* const red = lds;  // [kWaves][stride]
+  gc.flush(red + wave * stride, 0, lane);
+  go.flush(red + wave * stride, PP, lane);
+  {
+    const float s = dips_wave_sum(lsum);
+    if (lane == 0) red[wave * stride + PT] = s;
+  }
+  __syncthreads();
+  for (int q = threadIdx.x; q < stride; q += Cfg::kThreads) {
+    float s = 0.0f;
+    if (kGrad || q == PT) {
+#pragma unroll
+      for (int w = 0; w < Cfg::kWaves; ++w) s += red[w * stride + q];
+    }
+    const int64_t o = (int64_t)seg.row * stride + q;
+    gst(partial, o, seg.first ? s : gld(partial, o) + s);
+  }
+}
+
 template <int Lm, int Hm, int Lp, int Hp, bool kGrad, int PC1, int PC2, int Act>
 __device__ __forceinline__ void tile_step_body(const TileStepArgs& a, float* params, float* partial, int blk,
                                                int nblk, const TileSeg& seg) {
+  if constexpr (TileCfg<Lm, Hm, Lp, Hp, PC1>::kChain) {
+    tile_chain_body<Lm, Hm, kGrad, Act>(a, params, partial, blk, nblk, seg);
+    return;
+  } else {
   constexpr int kTileThreads = TileCfg<Lm, Hm, Lp, Hp, PC1>::kThreads;
   constexpr int kTileWaves = TileCfg<Lm, Hm, Lp, Hp, PC1>::kWaves;
   using NP = NetLayout<Lp, Hp>;
@@ -879,6 +1347,7 @@ __device__ __forceinline__ void tile_step_body(const TileStepArgs& a, float* par
     }
     const int64_t o = (int64_t)seg.row * stride + p;
     gst(partial, o, seg.first ? s : gld(partial, o) + s);
+  }
   }
 }
 
