@@ -366,24 +366,56 @@ struct HashGrad {
 // Buckets: appends (row, v0, v1) to the workgroup's slot of the row's bucket at
 // the workgroup's LDS cursor.
 //
-// Buckets are block-cyclic over groups of 64 consecutive rows: group G = row >>
-// 6 belongs to bucket G mod nb (nb a power of two), at local rows ((G / nb) <<
-// 6) + (row & 63) < kBRows.  The hot rows of the small dense levels thus spread
-// over many buckets, and a bucket still writes whole 512-byte row groups.
+// Buckets are block-cyclic over groups of consecutive rows, nb (a power of two) buckets: group G of the dense levels'
+// rows [0, dense), 4 rows a group, and group G of the hashed levels' rows, 64 a group, belong to bucket G mod nb, at
+// local rows G / nb groups into the bucket's dense or hashed part.  A workgroup's entries lie in one region, whose
+// rows on a dense level are few and adjacent: with groups of 64 rows there too, its slots of a few buckets overflowed
+// while the others were a third full, and 15% of the records went as atomic adds (backward of the 128^3 step, 65536
+// rows, 2^19-row levels: 512 us, now 377).  Four rows are the 32 bytes a bucket can write without reading (one row:
+// 352, but the sums 282 for 215 us); on the hashed levels 64 rows keep a line of entries in few slots (16 rows on
+// both kinds of level: 408 and 247 us).
+constexpr int kDShift = 2;
 constexpr int kGShift = 6;
-constexpr int kBRows = 8192;       // local rows of a bucket (LDS accumulator)
+constexpr int kBRows = 8192 + 68;  // local rows of a bucket (LDS accumulator): 8192 and the rounding of the two parts
 constexpr int kMaxBuckets = 4096;  // tables of up to 2^25 rows use the buckets
 
 struct BucketMap {
-  int shift;  // log2(nb)
-  __device__ __forceinline__ int bucket(int32_t row) const { return (row >> kGShift) & ((1 << shift) - 1); }
+  int shift;        // log2(nb)
+  int64_t dense;    // rows of the dense levels
+  int dense_local;  // local rows of a bucket's dense part
+  __host__ __device__ BucketMap(const HashLevels& H, int shift_) : shift(shift_), dense(H.rows) {
+    for (int l = H.L - 1; l >= 0; --l)
+      if (!H.res[l]) dense = H.offset[l];
+    dense_local = part(dense, kDShift);
+  }
+  // local rows of a part of n rows in groups of 2^g
+  __host__ __device__ int part(int64_t n, int g) const {
+    return (int)(((((n + (1 << g) - 1) >> g) + (1 << shift) - 1) >> shift) << g);
+  }
+  __host__ __device__ int local_rows(int64_t rows) const { return dense_local + part(rows - dense, kGShift); }
+  template <bool kDense>
+  __device__ __forceinline__ int bucket(int32_t row) const {
+    return (kDense ? row >> kDShift : (row - (int32_t)dense) >> kGShift) & ((1 << shift) - 1);
+  }
   __device__ __forceinline__ int local(uint32_t row) const {
-    return (int)(((row >> kGShift) >> shift) << kGShift) | (int)(row & ((1u << kGShift) - 1));
+    if (row < (uint32_t)dense) return (int)(((row >> kDShift) >> shift) << kDShift) | (int)(row & ((1u << kDShift) - 1));
+    const uint32_t h = row - (uint32_t)dense;
+    return dense_local + ((int)(((h >> kGShift) >> shift) << kGShift) | (int)(h & ((1u << kGShift) - 1)));
+  }
+  // table row of local row k of bucket b; rows or more where there is none
+  __device__ __forceinline__ int64_t row(int k, int b, int64_t rows) const {
+    if (k < dense_local) {
+      const int64_t r = ((((int64_t)(k >> kDShift) << shift) + b) << kDShift) + (k & ((1 << kDShift) - 1));
+      return r < dense ? r : rows;
+    }
+    k -= dense_local;
+    return dense + ((((int64_t)(k >> kGShift) << shift) + b) << kGShift) + (k & ((1 << kGShift) - 1));
   }
 };
 
 struct AtomicSink {
   float* gtab;
+  template <bool kDense>
   __device__ __forceinline__ void put(int32_t row, float v0, float v1) const {
     unsafeAtomicAdd(gtab + 2 * (int64_t)row, v0);
     unsafeAtomicAdd(gtab + 2 * (int64_t)row + 1, v1);
@@ -399,8 +431,9 @@ struct BucketSink {
   int cap;       // records a slot holds
   BucketMap map;
   float* gtab;
+  template <bool kDense>
   __device__ __forceinline__ void put(int32_t row, float v0, float v1) const {
-    const int b = map.bucket(row);
+    const int b = map.bucket<kDense>(row);
     const int pos = atomicAdd(cursor + b, 1);
     if (pos < cap) {
       slots[(int64_t)b * cap + pos] = make_uint4((uint32_t)row, __float_as_uint(v0), __float_as_uint(v1), 0u);
@@ -431,10 +464,10 @@ __device__ __forceinline__ void hash_scatter(const Sink& sink, int32_t row, floa
     const bool in = (same >> lane) & 1;
     const float s0 = dips_wave_sum(in ? v0 : 0.0f);
     const float s1 = dips_wave_sum(in ? v1 : 0.0f);
-    if (lane == leader) sink.put(key, s0, s1);
+    if (lane == leader) sink.template put<false>(key, s0, s1);
     rem &= ~same;
   }
-  if ((rem >> lane) & 1) sink.put(row, v0, v1);
+  if ((rem >> lane) & 1) sink.template put<false>(row, v0, v1);
 }
 
 // The 8 corner records of every lane in live on a dense (coarse) level, where a
@@ -462,7 +495,7 @@ __device__ __forceinline__ void hash_scatter_cell(const Sink& sink, const int32_
   for (int c = 0; c < 8; ++c) {
     const float s0 = dips_segmented_scan(on ? v0[c] : 0.0f, lane, head);
     const float s1 = dips_segmented_scan(on ? v1[c] : 0.0f, lane, head);
-    if (last) sink.put(rows[c], s0, s1);
+    if (last) sink.template put<true>(rows[c], s0, s1);
   }
 }
 
@@ -583,48 +616,88 @@ __global__ __launch_bounds__(kFwdThreads) void hash_fwd_kernel(HashArgs A, HashL
 // add runs ~9x the rate of a float32 one (measured: 1.8 T against 0.2 T lane
 // adds/s chip-wide, conflict-free float32 adds no faster), and it rounds less.
 constexpr int kBThreads = 1024;
-constexpr size_t kBucketLds = sizeof(double) * 2 * kBRows;  // 128 KB: one workgroup per CU
+// the two features of a table row at 4-byte alignment
+typedef float row2 __attribute__((ext_vector_type(2), aligned(4)));
+typedef __attribute__((address_space(1))) row2 global_row2;
+constexpr size_t kBucketLds = sizeof(double) * 2 * kBRows;  // 129 KB: one workgroup per CU
 __global__ __launch_bounds__(kBThreads) void hash_bucket_kernel(const uint4* __restrict__ recs,
                                                                 const int* __restrict__ cnt, int cap, int nb,
                                                                 BucketMap map, int64_t rows,
                                                                 float* __restrict__ gtab, float inv_b,
                                                                 float* __restrict__ gout,
                                                                 double* __restrict__ sq_part) {
-  extern __shared__ double bucket_acc[];  // 2 * kBRows
+  extern __shared__ double bucket_acc[];  // [kHF][kBRows]
   double* const acc = bucket_acc;
   __shared__ double wsum[kBThreads / DIPS_WAVE];
   const int b = blockIdx.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x / DIPS_WAVE;
-  for (int i = threadIdx.x; i < 2 * kBRows; i += kBThreads) acc[i] = 0.0;
+  const int nlocal = map.local_rows(rows);
+  for (int i = threadIdx.x; i < nlocal; i += kBThreads) acc[i] = acc[kBRows + i] = 0.0;
   __syncthreads();
-  // the slots of bucket b, one per backward workgroup, a wavefront each in turn
-  for (int blk = wave; blk < kHashBlocks; blk += kBThreads / DIPS_WAVE) {
-    const int n = cnt[(int64_t)b * kHashBlocks + blk];
-    const uint4* seg = recs + ((int64_t)blk * nb + b) * cap;
-    for (int i = lane; i < n; i += DIPS_WAVE) {
-      const uint4 rc = seg[i];
-      const int k = map.local(rc.x);
-      atomicAdd(acc + 2 * k, (double)__uint_as_float(rc.y));
-      atomicAdd(acc + 2 * k + 1, (double)__uint_as_float(rc.z));
-    }
+  // the slots of bucket b, one per backward workgroup, kSlotsPer of them to a wavefront.  Their record counts
+  // are read at once, and the next slot's first kAhead * 64 records before this slot's are added: the kernel waits
+  // for memory, for the records three quarters of its 215 us at the 128^3 step (0.3 GB); the LDS adds, hidden
+  // behind that, take 20.  16 lanes to a slot, four slots at once: 241 us.
+  constexpr int kSlotsPer = kHashBlocks / (kBThreads / DIPS_WAVE), kAhead = 4;
+  static_assert(kSlotsPer <= DIPS_WAVE, "slots of a wavefront");
+  const int sent = cnt[(int64_t)b * kHashBlocks + wave * kSlotsPer + min(lane, kSlotsPer - 1)];
+  const int counts = min(sent, cap);
+  auto slot = [&](int j) { return recs + ((int64_t)(wave * kSlotsPer + j) * nb + b) * cap; };
+  auto add = [&](const uint4& rc) {
+    const int k = map.local(rc.x);
+    atomicAdd(acc + k, (double)__uint_as_float(rc.y));
+    atomicAdd(acc + kBRows + k, (double)__uint_as_float(rc.z));
+  };
+  uint4 next[kAhead];
+  auto fetch = [&](int j) {
+    const int n = __builtin_amdgcn_readlane(counts, j);
+    const uint4* const seg = slot(j);
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q)
+      if (lane + q * DIPS_WAVE < n) next[q] = seg[lane + q * DIPS_WAVE];
+  };
+  fetch(0);
+#pragma unroll 1
+  for (int j = 0; j < kSlotsPer; ++j) {
+    const int n = __builtin_amdgcn_readlane(counts, j);
+    uint4 rc[kAhead];
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) rc[q] = next[q];
+    if (j + 1 < kSlotsPer) fetch(j + 1);
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q)
+      if (lane + q * DIPS_WAVE < n) add(rc[q]);
+    for (int i = lane + kAhead * DIPS_WAVE; i < n; i += DIPS_WAVE) add(slot(j)[i]);
   }
-  __syncthreads();
-  // local row k of group lg is table row ((lg * nb + b) << 6) + (k & 63); gtab holds
-  // the records past a slot's capacity.  Also the bucket's float64 sum of squares
-  // of the mean gradient inv_b * gtab (fixed order) for the clipping norm, and,
-  // when gout is given, that gradient.
+  const bool spilled = __syncthreads_or(sent > cap);
+  // gtab holds the records past a slot's capacity (zeros, not read, if there were none).  Also the bucket's float64
+  // sum of squares of the mean gradient inv_b * gtab (fixed order) for the clipping norm, and, when gout is given,
+  // that gradient.  kRows rows in flight a thread; with zeros read and one row at a time, 13 us more.
+  constexpr int kRows = 4;
   double v = 0.0;
-  for (int i = threadIdx.x; i < 2 * kBRows; i += kBThreads) {
-    const int k = i >> 1;
-    const int64_t g = ((int64_t)(k >> kGShift) << map.shift) + b;
-    const int64_t row = (g << kGShift) + (k & ((1 << kGShift) - 1));
-    if (row < rows) {
-      const int64_t idx = 2 * row + (i & 1);
-      const float tot = (float)((double)gtab[idx] + acc[i]);
-      gtab[idx] = tot;
-      const float gg = tot * inv_b;
-      if (gout) gout[idx] = gg;
-      v += (double)gg * (double)gg;
+  for (int k0 = threadIdx.x; k0 < nlocal; k0 += kRows * kBThreads) {
+    int64_t row[kRows];
+    row2 over[kRows];
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) {
+      const int k = k0 + q * kBThreads;
+      row[q] = k < nlocal ? map.row(k, b, rows) : rows;
+      over[q] = row2{0.0f, 0.0f};
+      if (spilled && row[q] < rows) over[q] = *(const global_row2*)(gtab + 2 * row[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) {
+      if (row[q] >= rows) continue;
+      const int k = k0 + q * kBThreads;
+      row2 tot, gg;
+#pragma unroll
+      for (int f = 0; f < kHF; ++f) {
+        tot[f] = (float)((double)over[q][f] + acc[f * kBRows + k]);
+        gg[f] = tot[f] * inv_b;
+        v += (double)gg[f] * (double)gg[f];
+      }
+      *(global_row2*)(gtab + 2 * row[q]) = tot;
+      if (gout) *(global_row2*)(gout + 2 * row[q]) = gg;
     }
   }
   v = dips_wave_sum_d(v);
@@ -770,9 +843,9 @@ __global__ __launch_bounds__(kHashThreads) void hash_bwd_kernel(HashArgs A, Hash
   const int stride = 2 * PM;
   __syncthreads();
   if constexpr (kBuckets) {
-    // records in this workgroup's slot of each bucket, bucket-major for the bucket sums
+    // records this workgroup sent to each bucket, bucket-major for the bucket sums
     for (int b = threadIdx.x; b < nb; b += kHashThreads)
-      cnt[(int64_t)b * kHashBlocks + blockIdx.x] = min(cursor[b], cap);
+      cnt[(int64_t)b * kHashBlocks + blockIdx.x] = cursor[b];
   }
   float* red = hash_lds + wave * stride;
   gp.flush(red, lane, E);
@@ -1180,10 +1253,9 @@ static int64_t hash_records(const HashLevels& H, int64_t nent) { return nent * H
 // the bucketed table gradient serves tables of up to kMaxBuckets buckets and
 // batches of fewer than 2^31 records; others use atomic adds
 static bool hash_bucketed(const HashLevels& H, int64_t nent, int* nb, int* shift = nullptr) {
-  // smallest power of two nb with nb * (kBRows / 64) row groups covering the table
-  const int64_t groups = (H.rows + (1 << kGShift) - 1) >> kGShift;
+  // smallest power of two nb whose buckets' local rows fit the accumulator
   int sh = 0;
-  while (((int64_t)kBRows >> kGShift << sh) < groups) ++sh;
+  while (sh < 16 && BucketMap(H, sh).local_rows(H.rows) > kBRows) ++sh;
   *nb = 1 << sh;
   if (shift) *shift = sh;
   return *nb <= kMaxBuckets && hash_records(H, nent) < INT_MAX;
@@ -1256,7 +1328,7 @@ int hash_step(const dips_grid_t* g, const dips_records_t* rec, const dips_mfma_b
   float* gvec = gtab + H.rows * kHF;
   int nb = 0, nb_shift = 0;
   const bool buckets = H.enc == 0 && hash_bucketed(H, nent, &nb, &nb_shift);
-  const BucketMap bmap{nb_shift};
+  const BucketMap bmap(H, nb_shift);
   const int cap = buckets ? hash_slot_cap(H, nent, nb) : 0;
   const int64_t nrec = buckets ? (int64_t)kHashBlocks * nb * cap : 0;
   float* encbuf = gvec + P;
