@@ -491,6 +491,24 @@ int dips_atoms_eval(const double* atoms, int32_t natoms, const int32_t* cell_sta
  * point (P000,P100,P101,P001,P010,P110,P011,P111); region (N,7) int8.
  * ------------------------------------------------------------------------- */
 
+/* Distinct positions of the 63 level-set samples of every grid node (7 stencil points, 8 corners of each one's
+ * cell).  t{x,y,z}[n][3][3]: per node of the axis, stencil sign e and corner sign c, the index of the coordinate
+ * node + e h + c h/2 among the axis' distinct coordinates (mx, my, at most 32 wz of them).
+ * mark: bits (mx my rows of wz words, zeroed by the caller) of the positions in use, count (mx my) set bits per row;
+ * pat: 4 rows of wz words, the z indices of all nodes with (e, c) = (0, 0), (0, +-1), (+-1, 0), (+-1, +-1).
+ * emit: with end = the inclusive sums of count, the positions in lattice order (pos, end[last] x 3 floats; ux, uy,
+ * uz: the distinct coordinates) and rank (as bits) of every word.
+ * gather: phis (N,7) and phic (N,7,8) from the values at these positions. */
+int dips_geom_lattice_mark(const int32_t* tx, const int32_t* ty, const int32_t* tz, int32_t nx, int32_t ny, int32_t nz,
+                           int64_t mx, int64_t my, int32_t wz, const uint32_t* pat, uint32_t* bits, int32_t* count,
+                           void* stream);
+int dips_geom_lattice_emit(const uint32_t* bits, int32_t nx, int32_t ny, int32_t nz, int64_t mx, int64_t my,
+                           int32_t wz, const int64_t* end, const float* ux, const float* uy, const float* uz,
+                           uint32_t* rank, float* pos, void* stream);
+int dips_geom_lattice_gather(const int32_t* tx, const int32_t* ty, const int32_t* tz, int32_t nx, int32_t ny,
+                             int32_t nz, int64_t mx, int64_t my, int32_t wz, const uint32_t* bits,
+                             const uint32_t* rank, const double* vals, double* phis, double* phic, void* stream);
+
 /* region[t] = 0 if cell t is crossed (0 < #(phi<0) < 8) else sign(phi(P000))
  * (per-point file :203-263), t over n7 = N*7 cells. */
 int dips_geom_regions(const double* phic, int64_t n7, int8_t* region, void* stream);

@@ -335,6 +335,45 @@ int dips_atoms_eval(const double* atoms, int32_t natoms, const int32_t* cell_sta
                       (hipStream_t)stream);
 }
 
+static bool lattice_args(int32_t nx, int32_t ny, int32_t nz, int64_t mx, int64_t my, int32_t wz) {
+  return nx >= 1 && ny >= 1 && nz >= 1 && (int64_t)nx * ny <= INT32_MAX && (int64_t)nx * ny * nz <= (1ll << 32) / 63 &&
+         mx >= 1 && mx <= 9ll * nx && my >= 1 && my <= 9ll * ny && wz >= 1 && wz <= (9ll * nz + 31) / 32 &&
+         (mx * my + 3) / 4 <= INT32_MAX;
+}
+
+int dips_geom_lattice_mark(const int32_t* tx, const int32_t* ty, const int32_t* tz, int32_t nx, int32_t ny, int32_t nz,
+                           int64_t mx, int64_t my, int32_t wz, const uint32_t* pat, uint32_t* bits, int32_t* count,
+                           void* stream) {
+  const Range range("K1 dips_geom_lattice_mark");
+  if (!lattice_args(nx, ny, nz, mx, my, wz) || !tx || !ty || !tz || !pat || !bits || !count) {
+    set_error("dips_geom_lattice_mark: invalid arguments");
+    return DIPS_EINVAL;
+  }
+  return geom_lattice_mark(tx, ty, tz, nx, ny, nz, mx, my, wz, pat, bits, count, (hipStream_t)stream);
+}
+
+int dips_geom_lattice_emit(const uint32_t* bits, int32_t nx, int32_t ny, int32_t nz, int64_t mx, int64_t my,
+                           int32_t wz, const int64_t* end, const float* ux, const float* uy, const float* uz,
+                           uint32_t* rank, float* pos, void* stream) {
+  const Range range("K1 dips_geom_lattice_emit");
+  if (!lattice_args(nx, ny, nz, mx, my, wz) || !bits || !end || !ux || !uy || !uz || !rank || !pos) {
+    set_error("dips_geom_lattice_emit: invalid arguments");
+    return DIPS_EINVAL;
+  }
+  return geom_lattice_emit(bits, mx, my, wz, end, ux, uy, uz, rank, pos, (hipStream_t)stream);
+}
+
+int dips_geom_lattice_gather(const int32_t* tx, const int32_t* ty, const int32_t* tz, int32_t nx, int32_t ny,
+                             int32_t nz, int64_t mx, int64_t my, int32_t wz, const uint32_t* bits,
+                             const uint32_t* rank, const double* vals, double* phis, double* phic, void* stream) {
+  const Range range("K1 dips_geom_lattice_gather");
+  if (!lattice_args(nx, ny, nz, mx, my, wz) || !tx || !ty || !tz || !bits || !rank || !vals || !phis || !phic) {
+    set_error("dips_geom_lattice_gather: invalid arguments");
+    return DIPS_EINVAL;
+  }
+  return geom_lattice_gather(tx, ty, tz, nx, ny, nz, my, wz, bits, rank, vals, phis, phic, (hipStream_t)stream);
+}
+
 int dips_geom_regions(const double* phic, int64_t n7, int8_t* region, void* stream) {
   const Range range("K1 dips_geom_regions");
   if (n7 < 0 || (n7 > 0 && (!phic || !region))) {

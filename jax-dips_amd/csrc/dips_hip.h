@@ -85,6 +85,13 @@ int opt_step_launch(const dips_net_t* net, const dips_opt_t* opt, const float* p
                     hipStream_t stream);
 
 // geom.hip
+int geom_lattice_mark(const int32_t* tx, const int32_t* ty, const int32_t* tz, int nx, int ny, int nz, int64_t mx,
+                      int64_t my, int wz, const uint32_t* pat, uint32_t* bits, int32_t* count, hipStream_t st);
+int geom_lattice_emit(const uint32_t* bits, int64_t mx, int64_t my, int wz, const int64_t* end, const float* ux,
+                      const float* uy, const float* uz, uint32_t* rank, float* pos, hipStream_t st);
+int geom_lattice_gather(const int32_t* tx, const int32_t* ty, const int32_t* tz, int nx, int ny, int nz, int64_t my,
+                        int wz, const uint32_t* bits, const uint32_t* rank, const double* vals, double* phis,
+                        double* phic, hipStream_t st);
 int geom_regions(const double* phic, int64_t n7, int8_t* region, hipStream_t st);
 int geom_cells(const dips_grid_t* g, float hx, float hy, float hz, const int32_t* cell_pt, int64_t ncell,
                const double* phic, double* vol_m, double* area_m, double* tri, double* tri_a, hipStream_t st);

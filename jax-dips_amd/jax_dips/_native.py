@@ -172,6 +172,12 @@ SIGNATURES = {
     "dips_atoms_eval": (ctypes.c_int, [_P, _I32, _P, _P, _I32, ctypes.c_double, ctypes.c_double, ctypes.c_double,
                                        ctypes.c_double, _P, _I64, _P, _P, _P]),
     "dips_geom_regions": (ctypes.c_int, [_P, _I64, _P, _P]),
+    "dips_geom_lattice_mark": (ctypes.c_int, [_P, _P, _P, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _I64, _I64,
+                                              ctypes.c_int32, _P, _P, _P, _P]),
+    "dips_geom_lattice_emit": (ctypes.c_int, [_P, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _I64, _I64,
+                                              ctypes.c_int32, _P, _P, _P, _P, _P, _P, _P]),
+    "dips_geom_lattice_gather": (ctypes.c_int, [_P, _P, _P, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _I64,
+                                                _I64, ctypes.c_int32, _P, _P, _P, _P, _P, _P]),
     "dips_geom_cells": (ctypes.c_int, [ctypes.POINTER(Grid), ctypes.c_float, ctypes.c_float, ctypes.c_float, _P, _I64,
                                        _P, _P, _P, _P, _P, _P]),
     "dips_geom_regression": (ctypes.c_int, [ctypes.POINTER(Grid), ctypes.c_float, ctypes.c_float, ctypes.c_float, _P,

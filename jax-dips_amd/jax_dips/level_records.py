@@ -97,6 +97,59 @@ def stencil_corner_phi(grid, S, ht, half, phi):
         tabs.append((U, inv.reshape(len(axv), 3, 3)))
     (Ux, Ix), (Uy, Iy), (Uz, Iz) = tabs
     My, Mz = Uy.numel(), Uz.numel()
+    phis = torch.empty((grid.npts, 7), dtype=torch.float64, device=device)
+    phic = torch.empty((grid.npts, 7, 8), dtype=torch.float64, device=device)
+    # on the GPU the distinct positions by a bit per lattice point (ranks in 32 bits), else by sorting keys; the
+    # same list in the same order
+    if device.type == "cuda" and 63 * ng < 2 ** 32:
+        _lattice_phi(grid.shape, tabs, phi, phis, phic)
+    else:
+        _sorted_phi(ng, tabs, phi, phis, phic)
+    if grid.npts > ng:
+        Se = S[ng:]
+        phis[ng:] = sample(phi, Se)
+        phic[ng:] = sample(phi, Se[:, :, None, :] + _offsets(CORNER_SIGNS, device)[None, None] * half)
+    return phis, phic
+
+
+def _lattice_phi(shape, tabs, phi, phis, phic):
+    """phi at the 63 samples of every grid node, once per distinct position
+    (dips_geom_lattice_*); tabs: per axis the distinct coordinates and the
+    nodes' indices (n, 3 stencil signs, 3 corner signs) into them."""
+    import torch
+
+    L, st = N.lib(), N.current_stream()
+    nx, ny, nz = (int(n) for n in shape)
+    (Ux, _), (Uy, _), (Uz, Iz) = tabs
+    device = Ux.device
+    Mx, My, wz = Ux.numel(), Uy.numel(), -(-Uz.numel() // 32)
+    tx, ty, tz = (i.to(torch.int32).contiguous() for _, i in tabs)
+    flags = torch.zeros((4, wz * 32), dtype=torch.int64, device=device)
+    for p, (es, cs) in enumerate((((1,), (1,)), ((1,), (0, 2)), ((0, 2), (1,)), ((0, 2), (0, 2)))):
+        flags[p, Iz[:, es][:, :, cs].reshape(-1)] = 1
+    pat = (flags.reshape(4, wz, 32) << torch.arange(32, device=device)).sum(2).to(torch.int32).contiguous()
+    bits = torch.zeros(Mx * My * wz, dtype=torch.int32, device=device)
+    count = torch.empty(Mx * My, dtype=torch.int32, device=device)
+    N.check(L.dips_geom_lattice_mark(N.ptr(tx), N.ptr(ty), N.ptr(tz), nx, ny, nz, Mx, My, wz, N.ptr(pat), N.ptr(bits),
+                                     N.ptr(count), st), "dips_geom_lattice_mark")
+    end = torch.cumsum(count, 0, dtype=torch.int64)
+    rank = torch.empty_like(bits)
+    pos = torch.empty((int(end[-1].item()), 3), dtype=torch.float32, device=device)
+    N.check(L.dips_geom_lattice_emit(N.ptr(bits), nx, ny, nz, Mx, My, wz, N.ptr(end), N.ptr(Ux), N.ptr(Uy), N.ptr(Uz),
+                                     N.ptr(rank), N.ptr(pos), st), "dips_geom_lattice_emit")
+    vals = sample(phi, pos).contiguous()
+    N.check(L.dips_geom_lattice_gather(N.ptr(tx), N.ptr(ty), N.ptr(tz), nx, ny, nz, Mx, My, wz, N.ptr(bits),
+                                       N.ptr(rank), N.ptr(vals), N.ptr(phis), N.ptr(phic), st),
+            "dips_geom_lattice_gather")
+
+
+def _sorted_phi(ng, tabs, phi, phis, phic):
+    """_lattice_phi by sorting the keys of all samples."""
+    import torch
+
+    (Ux, Ix), (Uy, Iy), (Uz, Iz) = tabs
+    My, Mz = Uy.numel(), Uz.numel()
+    device = Ux.device
     # keys of the 63 samples of every node: per stencil point e, the point (sign 0) then its 8 corners
     combos = [(e, c) for e in STENCIL for c in ((0, 0, 0),) + CORNER_SIGNS]
     keys = torch.empty((ng, len(combos)), dtype=torch.int64, device=device)
@@ -111,16 +164,8 @@ def stencil_corner_phi(grid, S, ht, half, phi):
     del uniq
     vals = sample(phi, pos)[inv].reshape(ng, 7, 9)
     del inv, pos
-    phis = torch.empty((grid.npts, 7), dtype=torch.float64, device=device)
-    phic = torch.empty((grid.npts, 7, 8), dtype=torch.float64, device=device)
     phis[:ng] = vals[:, :, 0]
     phic[:ng] = vals[:, :, 1:]
-    del vals
-    if grid.npts > ng:
-        Se = S[ng:]
-        phis[ng:] = sample(phi, Se)
-        phic[ng:] = sample(phi, Se[:, :, None, :] + _offsets(CORNER_SIGNS, device)[None, None] * half)
-    return phis.contiguous(), phic.contiguous()
 
 
 def build_level(grid, h, bounds, cbs, batch_size, device="cuda", coeffs=False):
