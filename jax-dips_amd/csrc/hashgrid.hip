@@ -400,9 +400,9 @@ struct BucketMap {
     return (int)(((((n + (1 << g) - 1) >> g) + (1 << shift) - 1) >> shift) << g);
   }
   __host__ __device__ int local_rows(int64_t rows) const { return dense_local + part(rows - dense, kGShift); }
-  template <bool kDense>
+  // by the row, not the level it was looked up on: a corner past a dense level's last node indexes the rows of the next
   __device__ __forceinline__ int bucket(int32_t row) const {
-    return (kDense ? row >> kDShift : (row - (int32_t)dense) >> kGShift) & ((1 << shift) - 1);
+    return (row < (int32_t)dense ? row >> kDShift : (row - (int32_t)dense) >> kGShift) & ((1 << shift) - 1);
   }
   __device__ __forceinline__ int local(uint32_t row) const {
     if (row < (uint32_t)dense) return (int)(((row >> kDShift) >> shift) << kDShift) | (int)(row & ((1u << kDShift) - 1));
@@ -422,7 +422,6 @@ struct BucketMap {
 
 struct AtomicSink {
   float* gtab;
-  template <bool kDense>
   __device__ __forceinline__ void put(int32_t row, float v0, float v1) const {
     unsafeAtomicAdd(gtab + 2 * (int64_t)row, v0);
     unsafeAtomicAdd(gtab + 2 * (int64_t)row + 1, v1);
@@ -438,9 +437,8 @@ struct BucketSink {
   int cap;       // records a slot holds
   BucketMap map;
   float* gtab;
-  template <bool kDense>
   __device__ __forceinline__ void put(int32_t row, float v0, float v1) const {
-    const int b = map.bucket<kDense>(row);
+    const int b = map.bucket(row);
     const int pos = atomicAdd(cursor + b, 1);
     if (pos < cap) {
       slots[(int64_t)b * cap + pos] = make_uint4((uint32_t)row, __float_as_uint(v0), __float_as_uint(v1), 0u);
@@ -471,10 +469,10 @@ __device__ __forceinline__ void hash_scatter(const Sink& sink, int32_t row, floa
     const bool in = (same >> lane) & 1;
     const float s0 = dips_wave_sum(in ? v0 : 0.0f);
     const float s1 = dips_wave_sum(in ? v1 : 0.0f);
-    if (lane == leader) sink.template put<false>(key, s0, s1);
+    if (lane == leader) sink.put(key, s0, s1);
     rem &= ~same;
   }
-  if ((rem >> lane) & 1) sink.template put<false>(row, v0, v1);
+  if ((rem >> lane) & 1) sink.put(row, v0, v1);
 }
 
 // The 8 corner records of every lane in live on a dense (coarse) level, where a
@@ -502,7 +500,7 @@ __device__ __forceinline__ void hash_scatter_cell(const Sink& sink, const int32_
   for (int c = 0; c < 8; ++c) {
     const float s0 = dips_segmented_scan(on ? v0[c] : 0.0f, lane, head);
     const float s1 = dips_segmented_scan(on ? v1[c] : 0.0f, lane, head);
-    if (last) sink.template put<true>(rows[c], s0, s1);
+    if (last) sink.put(rows[c], s0, s1);
   }
 }
 

@@ -17,6 +17,8 @@ TABLES = {
     "all dense": {"pos_levels": 3, "T": 2 ** 19, "N_min": 9, "N_max": 61},
     "first level hashed": {"pos_levels": 4, "T": 501, "N_min": 8, "N_max": 40},
     "many buckets": {"pos_levels": 12, "T": 2 ** 17, "N_min": 16, "N_max": 512},
+    # upper-face points index past the last dense level's rows, into the next level's; 256 slots a workgroup, none full
+    "past a dense level": {"pos_levels": 12, "T": 2 ** 17, "N_min": 16, "N_max": 540},
 }
 
 
