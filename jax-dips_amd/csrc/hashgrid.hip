@@ -377,10 +377,10 @@ struct HashGrad {
 // rows [0, dense), 4 rows a group, and group G of the hashed levels' rows, 64 a group, belong to bucket G mod nb, at
 // local rows G / nb groups into the bucket's dense or hashed part.  A workgroup's entries lie in one region, whose
 // rows on a dense level are few and adjacent: with groups of 64 rows there too, its slots of a few buckets overflowed
-// while the others were a third full, and 15% of the records went as atomic adds (backward of the 128^3 step, 65536
-// rows, 2^19-row levels: 512 us, now 377).  Four rows are the 32 bytes a bucket can write without reading (one row:
-// 352, but the sums 282 for 215 us); on the hashed levels 64 rows keep a line of entries in few slots (16 rows on
-// both kinds of level: 408 and 247 us).
+// while the others were part empty, and the atomic adds were a quarter of its memory requests (backward of the 128^3
+// step, 65536 rows, 2^19-row levels, 16-byte records: 512 us, then 377).  Four rows are the 32 bytes a bucket can
+// write without reading (one row: 352, but the sums 282 for 215 us); on the hashed levels 64 rows keep a line of
+// entries in few slots (16 rows on both kinds of level: 408 and 247 us).
 constexpr int kDShift = 2;
 constexpr int kGShift = 6;
 constexpr int kBRows = 8192 + 68;  // local rows of a bucket (LDS accumulator): 8192 and the rounding of the two parts
@@ -428,12 +428,19 @@ struct AtomicSink {
   }
 };
 
+// A record, one 12-byte store and load.  The records are most of the step's memory traffic, 33 to 41 M of them for 65536
+// rows of the 128^3 grid: at 16 bytes the backward took 377 us and the bucket sums 215, then 361 and 184.
+struct HashRecord {
+  uint32_t row;
+  float v0, v1;
+};
+
 // Records of one workgroup: bucket b's slot holds records [b * cap, (b + 1) * cap)
 // of `slots`; records past a slot's capacity go to gtab by atomic adds (gtab is
 // zeroed before the backward and the bucket sums add to it).
 struct BucketSink {
   int* cursor;   // LDS, per bucket: records this workgroup has sent to it
-  uint4* slots;  // records (row, v0 bits, v1 bits, 0): one 16-byte store each
+  HashRecord* slots;
   int cap;       // records a slot holds
   BucketMap map;
   float* gtab;
@@ -441,7 +448,7 @@ struct BucketSink {
     const int b = map.bucket(row);
     const int pos = atomicAdd(cursor + b, 1);
     if (pos < cap) {
-      slots[(int64_t)b * cap + pos] = make_uint4((uint32_t)row, __float_as_uint(v0), __float_as_uint(v1), 0u);
+      slots[(int64_t)b * cap + pos] = HashRecord{(uint32_t)row, v0, v1};
     } else {
       unsafeAtomicAdd(gtab + 2 * (int64_t)row, v0);
       unsafeAtomicAdd(gtab + 2 * (int64_t)row + 1, v1);
@@ -625,7 +632,7 @@ constexpr int kBThreads = 1024;
 typedef float row2 __attribute__((ext_vector_type(2), aligned(4)));
 typedef __attribute__((address_space(1))) row2 global_row2;
 constexpr size_t kBucketLds = sizeof(double) * 2 * kBRows;  // 129 KB: one workgroup per CU
-__global__ __launch_bounds__(kBThreads) void hash_bucket_kernel(const uint4* __restrict__ recs,
+__global__ __launch_bounds__(kBThreads) void hash_bucket_kernel(const HashRecord* __restrict__ recs,
                                                                 const int* __restrict__ cnt, int cap, int nb,
                                                                 BucketMap map, int64_t rows,
                                                                 float* __restrict__ gtab, float inv_b,
@@ -634,29 +641,31 @@ __global__ __launch_bounds__(kBThreads) void hash_bucket_kernel(const uint4* __r
   extern __shared__ double bucket_acc[];  // [kHF][kBRows]
   double* const acc = bucket_acc;
   __shared__ double wsum[kBThreads / DIPS_WAVE];
+  __shared__ int any_spilled;  // whether a slot of the bucket overflowed
   const int b = blockIdx.x;
+  if (threadIdx.x == 0) any_spilled = 0;
   const int lane = threadIdx.x & 63, wave = threadIdx.x / DIPS_WAVE;
   const int nlocal = map.local_rows(rows);
   for (int i = threadIdx.x; i < nlocal; i += kBThreads) acc[i] = acc[kBRows + i] = 0.0;
   __syncthreads();
   // the slots of bucket b, one per backward workgroup, kSlotsPer of them to a wavefront.  Their record counts
   // are read at once, and the next slot's first kAhead * 64 records before this slot's are added: the kernel waits
-  // for memory, for the records three quarters of its 215 us at the 128^3 step (0.3 GB); the LDS adds, hidden
-  // behind that, take 20.  16 lanes to a slot, four slots at once: 241 us.
+  // for memory, for the records three quarters of its time; the LDS adds are a tenth.  16 lanes to a slot, four
+  // slots at once: 241 us for 215 (16-byte records, 128^3 step).
   constexpr int kSlotsPer = kHashBlocks / (kBThreads / DIPS_WAVE), kAhead = 4;
   static_assert(kSlotsPer <= DIPS_WAVE, "slots of a wavefront");
   const int sent = cnt[(int64_t)b * kHashBlocks + wave * kSlotsPer + min(lane, kSlotsPer - 1)];
   const int counts = min(sent, cap);
   auto slot = [&](int j) { return recs + ((int64_t)(wave * kSlotsPer + j) * nb + b) * cap; };
-  auto add = [&](const uint4& rc) {
-    const int k = map.local(rc.x);
-    atomicAdd(acc + k, (double)__uint_as_float(rc.y));
-    atomicAdd(acc + kBRows + k, (double)__uint_as_float(rc.z));
+  auto add = [&](const HashRecord& rc) {
+    const int k = map.local(rc.row);
+    atomicAdd(acc + k, (double)rc.v0);
+    atomicAdd(acc + kBRows + k, (double)rc.v1);
   };
-  uint4 next[kAhead];
+  HashRecord next[kAhead];
   auto fetch = [&](int j) {
     const int n = __builtin_amdgcn_readlane(counts, j);
-    const uint4* const seg = slot(j);
+    const HashRecord* const seg = slot(j);
 #pragma unroll
     for (int q = 0; q < kAhead; ++q)
       if (lane + q * DIPS_WAVE < n) next[q] = seg[lane + q * DIPS_WAVE];
@@ -665,7 +674,7 @@ __global__ __launch_bounds__(kBThreads) void hash_bucket_kernel(const uint4* __r
 #pragma unroll 1
   for (int j = 0; j < kSlotsPer; ++j) {
     const int n = __builtin_amdgcn_readlane(counts, j);
-    uint4 rc[kAhead];
+    HashRecord rc[kAhead];
 #pragma unroll
     for (int q = 0; q < kAhead; ++q) rc[q] = next[q];
     if (j + 1 < kSlotsPer) fetch(j + 1);
@@ -674,7 +683,9 @@ __global__ __launch_bounds__(kBThreads) void hash_bucket_kernel(const uint4* __r
       if (lane + q * DIPS_WAVE < n) add(rc[q]);
     for (int i = lane + kAhead * DIPS_WAVE; i < n; i += DIPS_WAVE) add(slot(j)[i]);
   }
-  const bool spilled = __syncthreads_or(sent > cap);
+  if (sent > cap) any_spilled = 1;
+  __syncthreads();
+  const bool spilled = any_spilled != 0;
   // gtab holds the records past a slot's capacity (zeros, not read, if there were none).  Also the bucket's float64
   // sum of squares of the mean gradient inv_b * gtab (fixed order) for the clipping norm, and, when gout is given,
   // that gradient.  kRows rows in flight a thread; with zeros read and one row at a time, 13 us more.
@@ -725,7 +736,7 @@ __global__ __launch_bounds__(kHashThreads) void hash_bwd_kernel(HashArgs A, Hash
                                                                 const float* __restrict__ r_row,
                                                                 float* __restrict__ gtab,
                                                                 float* __restrict__ partial, int nb,
-                                                                int* __restrict__ cnt, uint4* __restrict__ recs,
+                                                                int* __restrict__ cnt, HashRecord* __restrict__ recs,
                                                                 int cap, BucketMap map) {
   extern __shared__ float hash_lds[];
   const int lane = threadIdx.x & 63;
@@ -1270,9 +1281,10 @@ static bool hash_bucketed(const HashLevels& H, int64_t nent, int* nb, int* shift
   return *nb <= kMaxBuckets && hash_records(H, nent) < INT_MAX;
 }
 
-// records a (workgroup, bucket) slot holds: the mean per slot if no entries
-// were aggregated (aggregation leaves about half), at least 64; records past it
-// take atomic adds.  DIPS_HASH_SLOT_CAP (read once per process) lowers it, so
+// records a (workgroup, bucket) slot holds: 4/3 of the mean per slot if no entries
+// were aggregated (aggregation leaves half to all of them), at least 64; records past it
+// take atomic adds.  At the mean itself the backward of the 128^3 step took 361 us for 316, the bucket sums,
+// which read the records that now arrive, 184 for 197.  DIPS_HASH_SLOT_CAP (read once per process) lowers it, so
 // that tests can run the atomic overflow path.
 static int hash_slot_cap(const HashLevels& H, int64_t nent, int nb) {
   static const int64_t forced = [] {
@@ -1281,7 +1293,7 @@ static int hash_slot_cap(const HashLevels& H, int64_t nent, int nb) {
   }();
   const int64_t slots = (int64_t)kHashBlocks * nb;
   const int64_t mean = (hash_records(H, nent) + slots - 1) / slots;
-  const int64_t cap = std::max<int64_t>(64, (mean + 15) / 16 * 16);
+  const int64_t cap = std::max<int64_t>(64, (mean * 4 / 3 + 15) / 16 * 16);
   return (int)(forced > 0 ? std::min(cap, forced) : cap);
 }
 
@@ -1296,7 +1308,7 @@ int64_t hash_workspace(const dips_hashgrid_t* hg, int64_t max_rows, int64_t max_
   int nb;
   n += max_nnz * (hash_width(H) + (H.enc == 0 ? kHW : 0));  // the forward's encodings (and activations)
   if (H.enc == 0 && hash_bucketed(H, max_nnz, &nb))
-    n += 4 * (int64_t)kHashBlocks * nb * hash_slot_cap(H, max_nnz, nb) + 4 + (int64_t)kHashBlocks * nb;
+    n += 3 * (int64_t)kHashBlocks * nb * hash_slot_cap(H, max_nnz, nb) + 4 + (int64_t)kHashBlocks * nb;
   return n;
 }
 
@@ -1328,7 +1340,7 @@ int hash_step(const dips_grid_t* g, const dips_records_t* rec, const dips_mfma_b
     set_error("hash step: too many parameters");
     return DIPS_EINVAL;
   }
-  // float workspace: u | r | MLP partial rows | table gradient | g | encodings | [record slots (16 B records,
+  // float workspace: u | r | MLP partial rows | table gradient | g | encodings | [record slots (12 B records,
   // kHashBlocks x nb slots of cap) | records per slot]
   float* u = work;
   float* r = u + nent;
@@ -1343,8 +1355,8 @@ int hash_step(const dips_grid_t* g, const dips_records_t* rec, const dips_mfma_b
   float* encbuf = gvec + P;
   float* rbase = encbuf + nent * (hash_width(H) + (H.enc == 0 ? kHW : 0));
   rbase += (4 - (reinterpret_cast<uintptr_t>(rbase) / sizeof(float)) % 4) % 4;  // 16-byte alignment
-  uint4* recs = reinterpret_cast<uint4*>(rbase);
-  int* cnt = reinterpret_cast<int*>(rbase + 4 * nrec);
+  HashRecord* recs = reinterpret_cast<HashRecord*>(rbase);
+  int* cnt = reinterpret_cast<int*>(rbase + 3 * nrec);
   const int nrb = rowsum_blocks(nrows);
   double* loss_part = dwork;
   double* sq_part = dwork + nrb;
