@@ -305,7 +305,7 @@ int dips_batch_steps(const dips_net_t* net, const dips_batch_plan_t* plan, int32
  * normals (m,3), the normal derivative grad u . n (m).  phase (m) uint8:
  * 1 -> Omega+ network (phi >= 0), 0 -> Omega- network.  Shapes of
  * dips_net_supported run one lane per point, those of dips_mfma_supported in
- * MFMA tiles of 16 points (grad u in forward mode).  Replaces
+ * MFMA tiles of 16 points (grad u by back-propagation).  Replaces
  * evaluate_solution_fn and the gradient post-processing of
  * evaluate_solution_and_gradients (trainer.py:836-844, :914-977). */
 int dips_eval(const dips_net_t* net, const float* params, const float* pts, const uint8_t* phase, const float* normals,
