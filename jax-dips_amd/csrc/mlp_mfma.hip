@@ -1619,9 +1619,11 @@ __global__ __launch_bounds__((EvalCfg<Lm, NBm, Lp, NBp, kGrad>::kThreads),
 mfma_eval_kernel(const float* __restrict__ params, int Hm, int Hp, EvalArgs E) {
   extern __shared__ __align__(16) float lds[];
   const int PPp = 4 * Hp + (Lp - 1) * (Hp * Hp + Hp) + Hp + 1;
-  eval_phase<Lp, NBp, kGrad, true>(E, params, FlatNet{Hp, Lp, 0}, lds);
-  __syncthreads();
-  eval_phase<Lm, NBm, kGrad, false>(E, params, FlatNet{Hm, Lm, PPp}, lds);
+  // gridDim.y 2: a workgroup per phase; 1: both, one after the other
+  const bool both = gridDim.y == 1;
+  if (both || blockIdx.y == 0) eval_phase<Lp, NBp, kGrad, true>(E, params, FlatNet{Hp, Lp, 0}, lds);
+  if (both) __syncthreads();
+  if (both || blockIdx.y == 1) eval_phase<Lm, NBm, kGrad, false>(E, params, FlatNet{Hm, Lm, PPp}, lds);
 }
 
 // loss = inv_b * sum of the row-sum partials (fixed order), gradient copy-out
@@ -1737,6 +1739,9 @@ int mfma_eval_launch(const dips_net_t* net, const float* params, const float* pt
   const int a = net->Lm, b = nb_of(Hm), c = net->Lp, d = nb_of(Hp);
   const int64_t ntiles = (m + 15) / 16;
   const EvalArgs E{pts, phase, nrm, m, u, grad, nrm ? gradn : nullptr};
+  // Where the tiles of both phases are resident at once, the phases go to workgroups of their own: a short launch is
+  // mostly the packing of a phase's weights (12^3 points, 3x64: 52 -> 27 us); in longer ones half of the workgroups
+  // would idle where one phase holds most points.
 #define Y(A, B, C, D, G)                                                                                         \
   {                                                                                                              \
     using Cfg = EvalCfg<A, B, C, D, G>;                                                                          \
@@ -1746,11 +1751,12 @@ int mfma_eval_launch(const dips_net_t* net, const float* params, const float* pt
                                  hipSuccess;                                                                     \
     (void)attr_set;                                                                                              \
     const int64_t waves = Cfg::kThreads / 64;                                                                    \
-    const int nblk = (int)std::min<int64_t>((ntiles + waves - 1) / waves,                                        \
-                                            resident_blocks((const void*)mfma_eval_kernel<A, B, C, D, G>,        \
-                                                            Cfg::kThreads, lds, 256));                           \
-    hipLaunchKernelGGL((mfma_eval_kernel<A, B, C, D, G>), dim3(nblk), dim3(Cfg::kThreads), lds, st, params, Hm,  \
-                       Hp, E);                                                                                   \
+    const int resident =                                                                                         \
+        resident_blocks((const void*)mfma_eval_kernel<A, B, C, D, G>, Cfg::kThreads, lds, 256);                  \
+    const int64_t want = (ntiles + waves - 1) / waves;                                                           \
+    const dim3 grid((unsigned)std::min<int64_t>(want, resident), 2 * want <= resident ? 2 : 1);                  \
+    hipLaunchKernelGGL((mfma_eval_kernel<A, B, C, D, G>), grid, dim3(Cfg::kThreads), lds, st, params, Hm, Hp,    \
+                       E);                                                                                       \
     return hip_status(hipGetLastError(), "mfma_eval_kernel launch");                                             \
   }
 #define X(A, B, C, D)                         \
