@@ -773,6 +773,7 @@ struct SplitStage {
   static constexpr int kInPart = 16 * 4;        // layer 0: the inputs' parts, [position][4], at the activations' place
   static constexpr int floats() { return kTile / 2; }
   static __device__ __forceinline__ int unit(int fb, int g, int p) { return 256 * fb + 64 * g + 4 * (p ^ (4 * (g >> 1))); }
+  static __device__ __forceinline__ int at(int f, int p) { return unit(f / 16, f % 16 / 4, p) + f % 4; }
 };
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef short s4v __attribute__((ext_vector_type(4)));
@@ -1113,6 +1114,33 @@ __device__ __forceinline__ void coop_backward(const float* __restrict__ W, const
   }
 }
 
+// a staged value from its parts, which lie `stride` halves apart.  An infinite value's second part is NaN (Inf - Inf):
+// its first part alone.
+__device__ __forceinline__ float split_value(const uint16_t* at, int stride) {
+  auto part = [&](int k) { return __uint_as_float((uint32_t)at[k * stride] << 16); };
+  const float h = part(0);
+  return isinf(h) ? h : (h + part(1)) + part(2);
+}
+
+// Whether delta feature f is infinite at a position of the group's tiles and NaN at none.  The feature's weight
+// gradients came out NaN then, as that position's second part is, and are formed again as float32 products: infinite.
+// Asked only where a sum has become NaN that was none.  64^3 points, a step: 665 us with and without; where the forward
+// pass is recomputed the branch's registers cost 2% (914 -> 934 us).
+template <int NB>
+__device__ __forceinline__ bool split_overflowed(const uint16_t* tiles, int f) {
+  using SS = SplitStage<NB>;
+  bool inf = false, nan = false;
+#pragma unroll 1
+  for (int s = 0; s < kBW; ++s)
+#pragma unroll 8
+    for (int p = 0; p < 16; ++p) {
+      const uint16_t h = tiles[s * SS::kTile + SS::kOperand + SS::at(f, p)];
+      inf |= (h & 0x7fff) == 0x7f80;
+      nan |= (h & 0x7fff) > 0x7f80;
+    }
+  return inf && !nan;
+}
+
 // coop_backward for the 64-wide networks: every contraction as split-bf16 products.  Per layer each wavefront
 // stages the parts of its tile's deltas (split once, for this and for the back-propagation) and activations; after
 // the barrier wavefront w contracts block (w / 2, w % 2) of 32 x 32 over the group's kBW tiles.  The products of a round go
@@ -1232,6 +1260,29 @@ __device__ __forceinline__ void split_backward(const float* __restrict__ W, cons
         t = mfma_bf32(a[0], b[0], t);
         __builtin_amdgcn_sched_barrier(0);  // one tile's operands at a time
       }
+      if (__any(t[0] != t[0] && G.dW[l - 1][0] == G.dW[l - 1][0])) {
+        int ln = lane;
+        asm volatile("" : "+v"(ln));  // no address of the rare branch is kept in registers from round to round
+        const int f = 32 * (wave % 2) + ln % 32, half = ln / 32;  // this lane's delta feature
+        if (split_overflowed<NB>(tiles, f)) {
+#pragma unroll 1
+          for (int q = -1; q < 16; ++q) {  // -1: the bias
+            float sum = 0.0f;
+#pragma unroll 1
+            for (int sp = 0; sp < 16 * kBW; ++sp) {
+              const uint16_t* A = tiles + sp / 16 * SS::kTile;
+              const float dv = split_value(A + SS::kOperand + SS::at(f, sp % 16), SS::kPart);
+              if (q >= 0)
+                sum = fmaf(split_value(A + SS::at(32 * (wave / 2) + 8 * (q / 4) + 4 * half + q % 4, sp % 16), SS::kPart), dv, sum);
+              else if (sp % 16 / 8 == half)
+                sum += dv;
+            }
+            if (q < 0) tb = sum;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) t[r] = r == q ? sum : t[r];
+          }
+        }
+      }
 #pragma unroll
       for (int q = 0; q < 16; ++q) G.dW[l - 1][q] += t[q];
       G.dB[l - 1] += tb;
@@ -1253,6 +1304,20 @@ __device__ __forceinline__ void split_backward(const float* __restrict__ W, cons
           b[p] = tr_read8(bp + lo, bp + hi);
         }
         t = bf6(a, b[0], b[1], b[2], t);
+      }
+      if (__any(t[0] != t[0] && G.dW0[0] == G.dW0[0])) {
+        int f = 16 * wave + i;
+        asm volatile("" : "+v"(f));
+        if (split_overflowed<NB>(tiles, f)) {
+          t = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+          for (int sp = 0; sp < 16 * kBW; ++sp) {
+            const uint16_t* A = tiles + sp / 16 * SS::kTile;
+            const float dv = split_value(A + SS::kOperand + SS::at(f, sp % 16), SS::kPart);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) t[r] = fmaf(split_value(A + 4 * (sp % 16) + r, SS::kInPart), dv, t[r]);
+          }
+        }
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) G.dW0[r] += t[r];

@@ -6,6 +6,7 @@ import pytest
 
 DIMS = (3, 64, 3, 64)
 P1 = 4 * 64 + 2 * (64 * 64 + 64) + 65  # parameters of one network
+LAYERS = {"W0": 0, "b0": 192, "W1": 256, "b1": 4352, "W2": 4416, "b2": 8512, "wo": 8576}
 
 
 def gradient(points, weight, const, plus, theta):
@@ -52,3 +53,37 @@ def test_products_have_no_common_sign():
         short += [g[o + 64 * k:o + 64 * k + 64] / (g[o + 192:o + 256] * float(xy[k])) - 1 for o in (0, P1) for k in (0, 1)]
     assert np.abs(short).max() <= 1e-6
     assert abs(np.mean(short)) <= 1.5e-8, np.mean(short)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layer,delta", [(2, np.inf), (1, 1.5e38), (0, 6e37)])
+def test_infinite_deltas(layer, delta):
+    """One row's deltas overflow float32 at a layer (delta: at the last one; a layer multiplies them by 3.7 here, the
+    factor of the packed weights among it): that layer's gradients of the row's network are infinite with the sign of their
+    products, as float32 products give them; the other network's stay finite."""
+    rng = np.random.default_rng(layer)
+    n, hot = 301, 147
+    pts = (0.2 + 0.6 * rng.random((n, 3))).astype(np.float32)
+    theta = np.zeros(2 * P1, np.float32)
+    for o in (0, P1):
+        theta[o:o + 192] = 0.4 * rng.uniform(-1, 1, 192)
+        theta[o + 256:o + 8512] = 0.02
+        for name in ("b1", "b2"):
+            theta[o + LAYERS[name]:o + LAYERS[name] + 64] = 0.1
+        theta[o + 8576:o + 8640] = 1.0
+    weight, const = 1 + rng.random(n), rng.normal(size=n)
+    a = pts[hot].astype(np.float64) @ theta[:192].reshape(3, 64).astype(np.float64)
+    acts = [np.tanh(a)]
+    for name in ("1", "2"):
+        acts.append(np.tanh(acts[-1] @ np.full((64, 64), float(np.float32(0.02))) + 0.1))
+    w = 1e20
+    u = acts[2].sum()
+    weight[hot] = w
+    const[hot] = 1e20 if np.isinf(delta) else delta / (w * (1 - acts[2][0] ** 2)) - w * u
+    plus = np.arange(n) % 2 == 1
+    g = gradient(pts, weight, const, plus, theta)
+    below = pts[hot] if layer == 0 else acts[layer - 1]
+    blk = g[LAYERS["W%d" % layer]:][:below.size * 64].reshape(-1, 64)
+    assert np.array_equal(blk, np.broadcast_to(np.copysign(np.inf, below)[:, None], blk.shape))
+    assert np.all(g[LAYERS["b%d" % layer]:][:64] == np.inf)
+    assert np.all(np.isfinite(g[P1:])) and np.any(g[P1:])
