@@ -649,39 +649,43 @@ __global__ __launch_bounds__(kBThreads) void hash_bucket_kernel(const HashRecord
   for (int i = threadIdx.x; i < nlocal; i += kBThreads) acc[i] = acc[kBRows + i] = 0.0;
   __syncthreads();
   // the slots of bucket b, one per backward workgroup, kSlotsPer of them to a wavefront.  Their record counts
-  // are read at once, and the next slot's first kAhead * 64 records before this slot's are added: the kernel waits
-  // for memory, for the records three quarters of its time; the LDS adds are a tenth.  16 lanes to a slot, four
-  // slots at once: 241 us for 215 (16-byte records, 128^3 step).
+  // are read at once, and the next kAhead * 64 records of a slot, or the next slot's first, before these are added: the
+  // kernel waits for memory, for the records three quarters of its time; the LDS adds are a tenth.  16 lanes to a
+  // slot, four slots at once: 241 us for 215 (16-byte records, 128^3 step).  With a slot's records past its first
+  // kAhead * 64 read 64 at a time as they are added: 843 us for 530 (8 levels of up to 2^15 rows in 32 buckets).
   constexpr int kSlotsPer = kHashBlocks / (kBThreads / DIPS_WAVE), kAhead = 4;
   static_assert(kSlotsPer <= DIPS_WAVE, "slots of a wavefront");
   const int sent = cnt[(int64_t)b * kHashBlocks + wave * kSlotsPer + min(lane, kSlotsPer - 1)];
   const int counts = min(sent, cap);
-  auto slot = [&](int j) { return recs + ((int64_t)(wave * kSlotsPer + j) * nb + b) * cap; };
   auto add = [&](const HashRecord& rc) {
     const int k = map.local(rc.row);
     atomicAdd(acc + k, (double)rc.v0);
     atomicAdd(acc + kBRows + k, (double)rc.v1);
   };
   HashRecord next[kAhead];
-  auto fetch = [&](int j) {
-    const int n = __builtin_amdgcn_readlane(counts, j);
-    const HashRecord* const seg = slot(j);
+  int j = 0, c = 0, n = __builtin_amdgcn_readlane(counts, 0);  // slot, first record of its chunk, records of the slot
+  auto fetch = [&] {
+    const HashRecord* const seg = recs + ((int64_t)(wave * kSlotsPer + j) * nb + b) * cap + c;
 #pragma unroll
     for (int q = 0; q < kAhead; ++q)
-      if (lane + q * DIPS_WAVE < n) next[q] = seg[lane + q * DIPS_WAVE];
+      if (lane + q * DIPS_WAVE < n - c) next[q] = seg[lane + q * DIPS_WAVE];
   };
-  fetch(0);
+  fetch();
 #pragma unroll 1
-  for (int j = 0; j < kSlotsPer; ++j) {
-    const int n = __builtin_amdgcn_readlane(counts, j);
+  while (j < kSlotsPer) {
+    const int left = n - c;
     HashRecord rc[kAhead];
 #pragma unroll
     for (int q = 0; q < kAhead; ++q) rc[q] = next[q];
-    if (j + 1 < kSlotsPer) fetch(j + 1);
+    c += kAhead * DIPS_WAVE;
+    if (c >= n) {
+      c = 0;
+      if (++j < kSlotsPer) n = __builtin_amdgcn_readlane(counts, j);
+    }
+    if (j < kSlotsPer) fetch();
 #pragma unroll
     for (int q = 0; q < kAhead; ++q)
-      if (lane + q * DIPS_WAVE < n) add(rc[q]);
-    for (int i = lane + kAhead * DIPS_WAVE; i < n; i += DIPS_WAVE) add(slot(j)[i]);
+      if (lane + q * DIPS_WAVE < left) add(rc[q]);
   }
   if (sent > cap) any_spilled = 1;
   __syncthreads();
@@ -1273,9 +1277,12 @@ static int64_t hash_records(const HashLevels& H, int64_t nent) { return nent * H
 // the bucketed table gradient serves tables of up to kMaxBuckets buckets and
 // batches of fewer than 2^31 records; others use atomic adds
 static bool hash_bucketed(const HashLevels& H, int64_t nent, int* nb, int* shift = nullptr) {
-  // smallest power of two nb whose buckets' local rows fit the accumulator
+  // Smallest power of two nb whose buckets' local rows fit the accumulator, then, for small tables, one that gives every
+  // CU a bucket to sum, while a slot keeps 64 records (its minimum: they grow by their rounding).  Steps of 65536 rows, with and
+  // without: 4 levels of up to 2^14 rows (256 or 8 buckets) 0.30 / 0.65 ms, 8 of 2^15 (256 or 32) 0.37 / 0.82 ms.
   int sh = 0;
   while (sh < 16 && BucketMap(H, sh).local_rows(H.rows) > kBRows) ++sh;
+  while (sh < 8 && (hash_records(H, nent) >> (sh + 1)) >= 64 * (int64_t)kHashBlocks) ++sh;
   *nb = 1 << sh;
   if (shift) *shift = sh;
   return *nb <= kMaxBuckets && hash_records(H, nent) < INT_MAX;
