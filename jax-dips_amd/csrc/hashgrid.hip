@@ -223,19 +223,31 @@ __device__ __forceinline__ void hash_encode(const HashLevels& H, const float* __
 // compiler from merging the loads of a column, and 960 of them, one per multiply-add, were the frequency
 // network's kernels (step of 65536 rows at 65^3: forward 168 -> 72 us, backward 224 -> 83; every unit still adds
 // its features in order).  With E a constant, and no guards, the loads move back into column order: 165 and 156.
-template <int N, typename WP>
+// kUnits: unit by unit, the same sums (hash_eval_kernel).
+template <bool kUnits = false, int N, typename WP>
 __device__ __forceinline__ float hash_mlp(WP W, int E, const float (&enc)[N], float (&act)[kHW]) {
-  float s[kHW];
+  if constexpr (kUnits) {
 #pragma unroll
-  for (int j = 0; j < kHW; ++j) s[j] = W[E * kHW + j];
+    for (int j = 0; j < kHW; ++j) {
+      float s = W[E * kHW + j];
 #pragma unroll
-  for (int k = 0; k < N; ++k)
-    if (k < E) {
-#pragma unroll
-      for (int j = 0; j < kHW; ++j) s[j] = fmaf(enc[k], W[k * kHW + j], s[j]);
+      for (int k = 0; k < N; ++k)
+        if (k < E) s = fmaf(enc[k], W[k * kHW + j], s);
+      act[j] = act_f<kActCelu>(s);
     }
+  } else {
+    float s[kHW];
 #pragma unroll
-  for (int j = 0; j < kHW; ++j) act[j] = act_f<kActCelu>(s[j]);
+    for (int j = 0; j < kHW; ++j) s[j] = W[E * kHW + j];
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      if (k < E) {
+#pragma unroll
+        for (int j = 0; j < kHW; ++j) s[j] = fmaf(enc[k], W[k * kHW + j], s[j]);
+      }
+#pragma unroll
+    for (int j = 0; j < kHW; ++j) act[j] = act_f<kActCelu>(s[j]);
+  }
   float u = W[E * kHW + 2 * kHW];
 #pragma unroll
   for (int j = 0; j < kHW; ++j) u = fmaf(act[j], W[E * kHW + kHW + j], u);
@@ -932,6 +944,12 @@ __global__ __launch_bounds__(256) void hash_zero_kernel(float* __restrict__ p, i
 static unsigned hash_zero_blocks(int64_t n) { return (unsigned)((n / 4 + 4 + 255) / 256); }
 
 // ---- evaluation: u and d u / d x ----------------------------------------------
+// Bound by the table gathers.  With a table beyond the L2s (8 x 4 MB) many points are evaluated faster with the MLP unit
+// by unit, whose long chain of single loads keeps fewer wavefronts gathering at once (kUnits / feature by feature, 16
+// levels of 2^19 rows: 160^3 points 6.05 / 6.47 ms, u alone 2.82 / 3.39; 90^3 1.14 / 1.11, 40^3 0.127 / 0.098);
+// smaller tables at every size feature by feature (16 levels of 2^14: 160^3 2.69 / 2.45).
+static bool hash_eval_units(const HashLevels& H, int64_t m) { return H.rows > (1 << 22) && m >= (1 << 19); }
+template <bool kUnits>
 __global__ __launch_bounds__(256) void hash_eval_kernel(HashLevels H, const float* __restrict__ params,
                                                         const float* __restrict__ pts,
                                                         const uint8_t* __restrict__ phase, int64_t m,
@@ -946,7 +964,7 @@ __global__ __launch_bounds__(256) void hash_eval_kernel(HashLevels H, const floa
   hash_pos(H, x, y, z, p);
   hash_encode(H, table, p, enc);
   const float* W = params + (phase[t] ? 0 : PM);
-  const float v = hash_mlp(W, E, enc, act);
+  const float v = hash_mlp<kUnits>(W, E, enc, act);
   u[t] = v;
   if (!grad) return;
   // d u / d enc_k = sum_j W0[k][j] Wout_j celu'(a_j)
@@ -1459,8 +1477,8 @@ int hash_eval(const dips_hashgrid_t* hg, const float* params, const float* pts, 
                        m, u, grad);
     return hip_status(hipGetLastError(), "freq_eval_kernel launch");
   }
-  hipLaunchKernelGGL(hash_eval_kernel, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, st, H, params, pts, phase, m,
-                     u, grad);
+  hipLaunchKernelGGL(hash_eval_units(H, m) ? hash_eval_kernel<true> : hash_eval_kernel<false>,
+                     dim3((unsigned)((m + 255) / 256)), dim3(256), 0, st, H, params, pts, phase, m, u, grad);
   return hip_status(hipGetLastError(), "hash_eval_kernel launch");
 }
 
