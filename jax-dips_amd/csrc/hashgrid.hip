@@ -944,11 +944,13 @@ __global__ __launch_bounds__(256) void hash_zero_kernel(float* __restrict__ p, i
 static unsigned hash_zero_blocks(int64_t n) { return (unsigned)((n / 4 + 4 + 255) / 256); }
 
 // ---- evaluation: u and d u / d x ----------------------------------------------
-// Bound by the table gathers.  With a table beyond the L2s (8 x 4 MB) many points are evaluated faster with the MLP unit
-// by unit, whose long chain of single loads keeps fewer wavefronts gathering at once (kUnits / feature by feature, 16
-// levels of 2^19 rows: 160^3 points 6.05 / 6.47 ms, u alone 2.82 / 3.39; 90^3 1.14 / 1.11, 40^3 0.127 / 0.098);
-// smaller tables at every size feature by feature (16 levels of 2^14: 160^3 2.69 / 2.45).
-static bool hash_eval_units(const HashLevels& H, int64_t m) { return H.rows > (1 << 22) && m >= (1 << 19); }
+// Bound by the table gathers.  With a table well beyond an L2 many points are evaluated faster with the MLP unit by
+// unit, whose long chain of single loads keeps fewer wavefronts gathering at once (kUnits / feature by feature, tables of
+// 6 M rows: 160^3 points 6.05 / 6.47 ms, u alone 2.82 / 3.39; 90^3 1.14 / 1.11, 40^3 0.127 / 0.098; 2.6 M rows: 220^3
+// 6.03 / 6.32, 128^3 1.09 / 1.02); up to 2 M rows at every size feature by feature (1.7 M: 220^3 9.83 / 9.56).
+static bool hash_eval_units(const HashLevels& H, int64_t m) {
+  return H.rows > (1 << 21) && m >= ((int64_t)1 << 43) / H.rows;
+}
 template <bool kUnits>
 __global__ __launch_bounds__(256) void hash_eval_kernel(HashLevels H, const float* __restrict__ params,
                                                         const float* __restrict__ pts,

@@ -1,5 +1,5 @@
 """dips_hash_eval has two loop orders of the MLP, chosen by the table's rows and the number of points: the same sums, so
-the same bits for the same points in calls on either side of the line (2^19 points, tables above 2^22 rows)."""
+the same bits for the same points in calls on either side of the line (rows times points: 2^43)."""
 import ctypes
 
 import pytest
@@ -14,10 +14,11 @@ def test_eval_bits_do_not_depend_on_the_call_size(levels):
 
     L = N.lib()
     hg = N.HashGrid(levels, 2, 1 << 19, 16, 2048, 1.0, 0)
-    assert L.dips_hash_table_rows(ctypes.byref(hg)) > 1 << 22
     g = torch.Generator().manual_seed(levels)
     theta = (0.2 * torch.randn(int(L.dips_hash_param_count(ctypes.byref(hg))), generator=g)).cuda()
-    m, part = (1 << 19) + 77, 1 << 18
+    m, part = 2000077, 1 << 19
+    rows = L.dips_hash_table_rows(ctypes.byref(hg))
+    assert rows * m >= 1 << 43 > rows * part
     pts = (2 * torch.rand(m, 3, generator=g) - 1).cuda()
     phase = (torch.rand(m, generator=g) < 0.5).to(torch.uint8).cuda()
 
