@@ -81,7 +81,7 @@ __global__ __launch_bounds__(kJudgeThreads) void grid_apply_kernel(
     const float* __restrict__ ent_w, int64_t nnz, const float* __restrict__ u, float* __restrict__ y, int with_c,
     const double* __restrict__ stop) {
   if (stop && *stop != 0.0) return;
-  __shared__ int4 rows[kJudgeThreads / DIPS_WAVE][DIPS_WAVE];  // point, first entry, end, whether no ghost is read
+  __shared__ int4 rows[kJudgeThreads / DIPS_WAVE][DIPS_WAVE];  // point, first entry, entries, whether no ghost is read
   __shared__ float2 wu[kJudgeThreads / DIPS_WAVE][DIPS_WAVE * (kApplyPer + 1)];  // per row, padded by one
   const int lane = threadIdx.x & (DIPS_WAVE - 1), wave = threadIdx.x / DIPS_WAVE;
   const int64_t back = (int64_t)gridDim.x - 1 - blockIdx.x, base = back / kRowGroup * kRowGroup, in = back - base;
@@ -89,35 +89,36 @@ __global__ __launch_bounds__(kJudgeThreads) void grid_apply_kernel(
       base + kRowGroup <= (int64_t)gridDim.x ? base + (in % kXcds) * (kRowGroup / kXcds) + in / kXcds : back;
   const int64_t row = blk * kJudgeThreads + threadIdx.x;
   const int64_t npts = (int64_t)nx * ny * nz;
-  int pt = -1, beg = 0, end = 0;
+  int pt = -1, beg = 0;
+  uint32_t len = 0;  // entries are counted from their row's first: entry indices go up to the largest int
   if (row < nrows) {
     pt = row_point[row];
     beg = max(row_ptr[row], 0);
-    end = (int)min((int64_t)row_ptr[row + 1], nnz);
+    len = (uint32_t)max(min((int64_t)row_ptr[row + 1], nnz) - beg, (int64_t)0);
   }
   const bool on = pt >= 0 && pt < npts;
-  if (!on) end = beg;
+  if (!on) len = 0;
   {
     // two nodes inside the grid (three below the top of the last axis: codes 125..127, outside the 5^3 cube,
     // decode to 3 there)
     const int k = pt % nz, ij = pt / nz, j = ij % ny, i = ij / ny;
     const bool inner = on && i >= 2 && i < nx - 2 && j >= 2 && j < ny - 2 && k >= 2 && k < nz - 3;
-    rows[wave][lane] = make_int4(pt, beg, end, inner ? 1 : 0);
+    rows[wave][lane] = make_int4(pt, beg, (int)len, inner ? 1 : 0);
   }
   float acc = (on && with_c) ? row_c[row] : 0.0f;
   const int sub = lane % kApplyPer, slot = lane / kApplyPer;
   __builtin_amdgcn_wave_barrier();
-  for (int c0 = 0; __any(beg + c0 < end); c0 += kApplyPer) {
+  for (uint32_t c0 = 0; __any(c0 < len); c0 += kApplyPer) {
     int4 rw[kApplyPasses];
     uint32_t code[kApplyPasses];
     float w[kApplyPasses], v[kApplyPasses];
 #pragma unroll
     for (int q = 0; q < kApplyPasses; ++q) {
       rw[q] = rows[wave][q * kPassRows + slot];
-      const int e = rw[q].y + c0 + sub;
       code[q] = 0;
       w[q] = 0.0f;
-      if (e < rw[q].z) {
+      if (c0 + sub < (uint32_t)rw[q].z) {
+        const uint32_t e = (uint32_t)rw[q].y + c0 + sub;
         code[q] = ent_code[e];
         w[q] = ent_w[e];
       }
@@ -125,7 +126,7 @@ __global__ __launch_bounds__(kJudgeThreads) void grid_apply_kernel(
 #pragma unroll
     for (int q = 0; q < kApplyPasses; ++q) {
       v[q] = 0.0f;
-      if (rw[q].y + c0 + sub < rw[q].z) {
+      if (c0 + sub < (uint32_t)rw[q].z) {
         if (rw[q].w) {
           int ox, oy, oz;
           dips_decode_offset(code[q], ox, oy, oz);
@@ -143,7 +144,7 @@ __global__ __launch_bounds__(kJudgeThreads) void grid_apply_kernel(
 #pragma unroll
     for (int q = 0; q < kApplyPer; ++q) {
       const float2 p = wu[wave][lane * (kApplyPer + 1) + q];
-      if (beg + c0 + q < end) acc = fmaf(p.x, p.y, acc);
+      if (c0 + q < len) acc = fmaf(p.x, p.y, acc);
     }
     __builtin_amdgcn_wave_barrier();
   }
