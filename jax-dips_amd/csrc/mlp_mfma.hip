@@ -1790,8 +1790,8 @@ int64_t mfma_workspace_floats(const dips_net_t* n, int64_t max_rows, int64_t max
 }
 
 // Workgroups of a persistent kernel resident at once on the current device
-// (compute units x occupancy), looked up once per kernel and device; fallback
-// if the runtime cannot say.  A persistent grid of exactly this size runs in
+// (compute units x occupancy), looked up once per kernel and device, whose LDS limit
+// for the kernel is raised to lds first; fallback if the runtime cannot say.  A persistent grid of exactly this size runs in
 // one wave of workgroups, so no workgroup starts after others have finished.
 int resident_blocks(const void* fn, int threads, size_t lds, int fallback) {
   static std::mutex mu;
@@ -1803,6 +1803,7 @@ int resident_blocks(const void* fn, int threads, size_t lds, int fallback) {
     if (e.first.first == fn && e.first.second == dev) return e.second;
   int per_cu = 0, cus = 0;
   int n = fallback;
+  (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, lds) == hipSuccess &&
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && per_cu > 0 && cus > 0)
     n = per_cu * cus;
@@ -1829,10 +1830,6 @@ int mfma_eval_launch(const dips_net_t* net, const float* params, const float* pt
   {                                                                                                              \
     using Cfg = EvalCfg<A, B, C, D, G>;                                                                          \
     constexpr size_t lds = sizeof(float) * Cfg::kFloats;                                                         \
-    static const bool attr_set = hipFuncSetAttribute((const void*)mfma_eval_kernel<A, B, C, D, G>,               \
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) ==    \
-                                 hipSuccess;                                                                     \
-    (void)attr_set;                                                                                              \
     const int64_t waves = Cfg::kThreads / 64;                                                                    \
     const int resident =                                                                                         \
         resident_blocks((const void*)mfma_eval_kernel<A, B, C, D, G>, Cfg::kThreads, lds, 256);                  \
