@@ -6,6 +6,7 @@ are passed as raw pointers (torch tensors are used only to own device memory
 and to name the current HIP stream).
 """
 import ctypes
+import hashlib
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -204,6 +205,18 @@ def lib():
             fn.argtypes = args
         _lib = L
     return _lib
+
+
+_revision = None
+
+
+def library_revision():
+    """Hash of the native library's file: what was measured with one build does not hold for another."""
+    global _revision
+    if _revision is None:
+        with open(LIB_PATH, "rb") as f:
+            _revision = hashlib.sha256(f.read()).hexdigest()[:16]
+    return _revision
 
 
 _roctx = None

@@ -723,22 +723,34 @@ class BatchEngine:
             for t, v in zip((e.params, e.m, e.v, e.count, e.loss_hist), s):
                 t.copy_(v)
 
+    def _autotune_key(self, grids, recs):
+        import hashlib
+        import json
+
+        import torch
+
+        arch = torch.cuda.get_device_properties(torch.cuda.current_device()).gcnArchName
+        sizes = sorted((int(g.npts), int(r.batch_size), np.diff(r.tiles(g)["batch_tile_begin"]).tolist())
+                       for g, r in zip(grids, recs))
+        net = [int(self.net.Lm), int(self.net.Hm), int(self.net.Lp), int(self.net.Hp), int(self.net.pc_w1),
+               int(self.net.pc_w2), int(self.net.act)]
+        return json.dumps([arch, N.library_revision(), net, [s[:2] for s in sizes],
+                           hashlib.sha256(json.dumps(sizes).encode()).hexdigest()[:16]])
+
     def autotune(self, grids, recs, caps=(256, 128, 64, 32, 16), steps=6, cache_path=None):
         """Choose the batched step's shape (dips_batch_cfg_t: blocks per
         problem and step, persistent grid size) by timing `steps` global steps
         of these records for every candidate, from the same state (restored
-        after each).  Results are cached in memory and in a JSON file keyed by
-        (GPU architecture, network shape, the problems' point counts and batch
-        sizes); returns the chosen (blk_cap, grid_blocks)."""
+        after each), while every problem still trains.  Results are cached in
+        memory and in a JSON file keyed by (GPU architecture, native library,
+        network shape, the problems' point counts, batch sizes and tiles per
+        batch); returns the chosen (blk_cap, grid_blocks)."""
         import json
         import os
 
         import torch
 
-        arch = torch.cuda.get_device_properties(torch.cuda.current_device()).gcnArchName
-        sizes = sorted((int(g.npts), int(r.batch_size)) for g, r in zip(grids, recs))
-        key = json.dumps([arch, [int(self.net.Lm), int(self.net.Hm), int(self.net.Lp), int(self.net.Hp),
-                                 int(self.net.pc_w1), int(self.net.pc_w2), int(self.net.act)], sizes])
+        key = self._autotune_key(grids, recs)
         path = cache_path or os.environ.get("DIPS_AUTOTUNE_CACHE",
                                             os.path.join(os.path.expanduser("~"), ".cache", "jax_dips_amd",
                                                          "batch_autotune.json"))
@@ -753,12 +765,14 @@ class BatchEngine:
             _BATCH_TUNED[key] = tuple(disk[key]["cfg"])
             return _BATCH_TUNED[key]
         snap = self._snapshot()
+        # epochs for the warm-up step and the timed ones: a step past a problem's last does nothing for it
+        epochs = -(-(int(steps) + 1) // min(len(r.batch_begin) for r in recs))
         # persistent grids of one and two workgroups per resident slot
-        resident = int(self.setup(grids, recs, 1, (0, 0)).grid_blocks)
+        resident = int(self.setup(grids, recs, epochs, (0, 0)).grid_blocks)
         timings = {}
         for cap in caps:
             for grid in (resident, 2 * resident):
-                plan = self.setup(grids, recs, 1, (cap, grid))
+                plan = self.setup(grids, recs, epochs, (cap, grid))
                 self.steps(plan, 1)  # warm-up
                 ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
                 ev[0].record()
