@@ -280,7 +280,8 @@ typedef struct {
 /* Host record of a set-up batched run, for dips_batch_steps. */
 typedef struct {
   int32_t nprob;        /* problems */
-  int32_t nitems;       /* work items per global step */
+  int32_t nitems;       /* sum over the problems of their most blocks (>= 1); the items of a step, blocks or parts of
+                           blocks of the problems still running, are decided on the device */
   int32_t blk_cap;
   int32_t grid_blocks;
   int32_t max_steps;    /* global steps of the nepochs epochs (max over problems of nepochs * nbatches) */

@@ -163,7 +163,8 @@ __device__ __forceinline__ void tile_forward(const float* __restrict__ W, float 
 }
 
 // ---- hidden layers on the bf16 matrix cores, to float32 accuracy --------------
-// Each float32 operand x is split exactly into three bf16 parts by truncation:
+// Each float32 operand x is split exactly into three bf16 parts by truncation (the backward's staged operands and
+// the evaluation's weights with rounded parts: bf_split_near, bf_part):
 // x0 = x with the low 16 bits cleared, x1 likewise of x - x0, x2 = x - x0 - x1
 // (x has 24 significant bits, each part holds 8: x0 + x1 + x2 == x bit for bit
 // for normal x, |x1| < 2^-7 |x|, |x2| < 2^-15 |x|).  A product a w is then the
@@ -317,7 +318,7 @@ __device__ void pack_weights_bf(const float* __restrict__ params, FlatNet fn, fl
   }
   uint32_t* wb = reinterpret_cast<uint32_t*>(lds + PK::nf());
   // a pair of weights at a time, all three parts of it, several pairs' loads in flight: part by part, each waiting for its
-  // own loads, this was a third of a one-round launch (3x64, 23^3 points: step 107 -> 90 us, evaluation 27 -> 16)
+  // own loads, this was a third of a one-round launch (3x64, 23^3 points: step 107 -> 88 us, evaluation 27 -> 16)
 #pragma unroll 4
   for (int d = threadIdx.x; d < 4 * PK::units() / 3; d += blockDim.x) {
     const int u = d % 4, lane = (d / 4) % 64;
@@ -1147,9 +1148,10 @@ __device__ __forceinline__ bool split_overflowed(const uint16_t* tiles, int f) {
 // to a fresh accumulator that is then added to the running one: one rounding at the running sum's size per round.
 // Error of a step's gradient against 64 bits (2-norm, mean of three seeds; float32 MFMA / truncated splits / these):
 // star 23^3 1.38e-7 / 1.54e-7 / 1.24e-7, Poisson-Boltzmann 256^3 3.5e-6 / 1.13e-7 / 0.92e-7.
-// Bound by the matrix and VALU cycles together (beside VALU work a bf16 MFMA still costs most of its own).  At 128^3
-// (star, last zoom level, 110 K tiles per batch): 619 -> 500 us against the same contraction in float32 MFMA, which
-// takes 2.7x the matrix cycles, during which the SIMD issues no VALU work at all.  Splitting with v_dot2 (7 instructions a
+// Bound by the matrix and VALU cycles together (beside VALU work a bf16 MFMA still costs most of its own): each is busy
+// 36% of the SIMD cycles, 8% of them at once; the wavefronts wait for LDS and each other a third of theirs.  At 128^3
+// (star, last zoom level, 110 K tiles per batch): 619 -> 500 us against the same contraction in float32 MFMA, which takes
+// 2.7x the matrix cycles, during which the SIMD issues no VALU work at all.  Splitting with v_dot2 (7 instructions a
 // pair instead of 11): 2% slower, it does not run beside the MFMA either.
 template <int L, int NB, class Prefetch>
 __device__ __forceinline__ void split_backward(const float* __restrict__ W, const float* __restrict__ wor, float seed,
@@ -1273,7 +1275,8 @@ __device__ __forceinline__ void split_backward(const float* __restrict__ W, cons
               const uint16_t* A = tiles + sp / 16 * SS::kTile;
               const float dv = split_value(A + SS::kOperand + SS::at(f, sp % 16), SS::kPart);
               if (q >= 0)
-                sum = fmaf(split_value(A + SS::at(32 * (wave / 2) + 8 * (q / 4) + 4 * half + q % 4, sp % 16), SS::kPart), dv, sum);
+                sum = fmaf(split_value(A + SS::at(32 * (wave / 2) + 8 * (q / 4) + 4 * half + q % 4, sp % 16),
+                                       SS::kPart), dv, sum);
               else if (sp % 16 / 8 == half)
                 sum += dv;
             }
@@ -1328,10 +1331,10 @@ __device__ __forceinline__ void split_backward(const float* __restrict__ W, cons
 }
 
 // Groups of kBW wavefronts per backward workgroup, each with tiles, stage and partial rows of its own.  With a
-// 64-wide network a workgroup has two, which share the back-propagation weights (48 KB; with two stages of 54 KB
-// one workgroup fills a CU's LDS); the second runs one barrier behind the first, so that between any two barriers one group stages
-// and back-propagates (VALU) while the other contracts (matrix cores, LDS).  The recomputing variant, which also holds the
-// forward copy, has room for one; a group's tiles and sums are the same either way.
+// 64-wide network a workgroup has two, which share the back-propagation weights (48 KB; with two stages of 48 KB
+// one workgroup fills a CU's LDS); the second runs one barrier behind the first, so that between any two barriers one
+// group stages and back-propagates (VALU) while the other contracts (matrix cores, LDS).  The recomputing variant, which
+// also holds the forward copy, has room for one; a group's tiles and sums are the same either way.
 template <int NBm, int NBp, bool kStored>
 constexpr int bwd_groups() {
   return kStored && (NBm == 4 || NBp == 4) ? 2 : 1;
@@ -1581,7 +1584,7 @@ __global__ void count_inc_kernel(int32_t* count) {
 // ---- evaluation at arbitrary points: u and grad_x u --------------------------------
 // The training step's tile passes: the forward pass in FwdPack's copy and, for grad u, one
 // back-propagation of d u / d u = 1 down to the inputs (kGrad) in the backward's copy; u alone otherwise.  Bound by
-// the matrix and VALU work of those two passes.  3x64 at 256^3 points with grad u: 3.7 ms; value and three input
+// the matrix and VALU work of those two passes.  3x64 at 256^3 points with grad u: 3.6 ms; value and three input
 // tangents propagated forward together in float32 MFMA: 10.4 ms (four chains of products instead
 // of two, each 2.7x the matrix cycles of the split-bf16 ones).
 // A workgroup packs the + network, takes its tiles of 16 consecutive points that hold a + point, then the same for
@@ -1598,7 +1601,7 @@ struct EvalCfg {
   static constexpr int kP = EvalPhase<Lp, NBp, kGrad>::floats(), kM = EvalPhase<Lm, NBm, kGrad>::floats();
   static constexpr int kFloats = kP > kM ? kP : kM;
   // Where the copies take more than half of the LDS (3x64 with grad u, 100 KB) one workgroup of 12 wavefronts with
-  // 168 registers each (256^3 points: 3.70 ms; 16 of 128, which spill: 4.85; 8 of 256: 4.16), else
+  // 168 registers each (256^3 points, in one build: 3.70 ms; 16 of 128, which spill: 4.85; 8 of 256: 4.16), else
   // workgroups of 8, six wavefronts per SIMD for u alone (1.75 ms; four: 1.94).
   static constexpr bool kWide = kFloats * sizeof(float) > 80 * 1024;
   static constexpr int kThreads = kWide ? 768 : 512;
@@ -1824,7 +1827,7 @@ int mfma_eval_launch(const dips_net_t* net, const float* params, const float* pt
   const int64_t ntiles = (m + 15) / 16;
   const EvalArgs E{pts, phase, nrm, m, u, grad, nrm ? gradn : nullptr};
   // Where the tiles of both phases are resident at once, the phases go to workgroups of their own: a short launch is
-  // mostly the packing of a phase's weights (12^3 points, 3x64: 52 -> 27 us); in longer ones half of the workgroups
+  // mostly the packing of a phase's weights (12^3 points, 3x64: 28 -> 16 us); in longer ones half of the workgroups
   // would idle where one phase holds most points.
 #define Y(A, B, C, D, G)                                                                                         \
   {                                                                                                              \
