@@ -107,7 +107,8 @@ typedef const __attribute__((address_space(1))) row4 global_row4;
 // A lane owns four neighbouring parameters (16-byte loads of a row) and a group of wavefronts every kGroups-th row;
 // the groups' sums meet in LDS and are added in order.  The kernel is a latency chain (rows -> norm ->
 // update) on one CU; with a wavefront's lanes over the rows instead, the float64 exchange between the lanes of every
-// parameter was most of it: 20.7 -> 7.2 us (32 rows of 707), 11.7 -> 8.0 us (256 of 420), 6.3 -> 5.9 us (256 of 168).
+// parameter was most of it: 18.4 -> 11.4 us (256 rows of 707), 11.6 -> 7.5 us (of 420), 6.2 -> 5.4 us (of 168).
+// The schedule's powf between the loads and the sums: 0.4 to 1.4 us of that (after the sums, every wavefront waited for it).
 // kGroups depends on the shape only, so that every launch form adds in the same order.
 template <int kStride, int kTileWaves>
 __device__ void tile_reduce_apply(const float* partial, int nblk, int nseg, const FusedOpt& fo, float* params) {
@@ -118,7 +119,7 @@ __device__ void tile_reduce_apply(const float* partial, int nblk, int nseg, cons
   constexpr int kGroups = 16 / kRowWaves;
   constexpr int kTeams = kTileWaves / kRowWaves;  // groups at work at once
   static_assert(kStride >= 4 && kRowWaves <= 8 && kRowWaves <= kTileWaves, "partial row width");
-  __shared__ double gsum[kGroups][kStride];
+  __shared__ double gsum[kStride <= kTileWaves ? 1 : kGroups][kStride];
   __shared__ float gsh[kStride];
   __shared__ double dred[kTileWaves];
   __shared__ float sched[3];
@@ -138,53 +139,80 @@ __device__ void tile_reduce_apply(const float* partial, int nblk, int nseg, cons
     vv[q] = gld(fo.v, pc);
   }
   const int c = gld(fo.count, 0);
-  const int col = min(4 * (wave % kRowWaves * DIPS_WAVE + lane), kStride - 4);
-  for (int g = wave / kRowWaves; g < kGroups && wave < kTeams * kRowWaves; g += kTeams) {
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    // 16 rows in flight: of 16 blocks, or of 4 blocks in kSegs parts each
-    auto add = [&](auto segs) {
-      constexpr int kS = decltype(segs)::value, kChunk = 16 / kS;
-      for (int b0 = g; b0 < nblk; b0 += kChunk * kGroups) {
-        row4 v[kChunk][kS];
+  // step-dependent scalars, computed once by the last wavefront (powf is long) while its rows are loaded
+  bool sched_due = wave == kTileWaves - 1;
+  auto schedule = [&] {
+    if (sched_due && lane == 0) {
+      const float t1 = (float)(c + 1);
+      sched[0] = schedule_lr(fo.opt, c);
+      sched[1] = 1.0f - powf(0.9f, t1);
+      sched[2] = 1.0f - powf(0.999f, t1);
+    }
+    sched_due = false;
+  };
+  if constexpr (kStride <= kTileWaves) {
+    // A wavefront per parameter, its lanes over the rows: a row's few 16-byte pieces would leave most lanes of a
+    // load idle and take as many loads as there are rows (256 rows of 13: 5.2 us, like this 3.4).
+    if (wave < kStride) {
+      float v[kMaxTileBlocks / DIPS_WAVE];
 #pragma unroll
-        for (int j = 0; j < kChunk; ++j)
-#pragma unroll
-          for (int k = 0; k < kS; ++k)
-            v[j][k] =
-                *(global_row4*)(partial + ((int64_t)min(b0 + j * kGroups, nblk - 1) * kS + k) * kStride + col);
-#pragma unroll
-        for (int j = 0; j < kChunk; ++j)
-          if (b0 + j * kGroups < nblk) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              float t = v[j][0][i];
-#pragma unroll
-              for (int k = 1; k < kS; ++k) t += v[j][k][i];
-              acc[i] += (double)t;
-            }
-          }
+      for (int i = 0; i < kMaxTileBlocks / DIPS_WAVE; ++i) {
+        const int64_t row = (int64_t)min(lane + i * DIPS_WAVE, nblk - 1) * nseg;
+        v[i] = gld(partial, row * kStride + wave);
+        for (int k = 1; k < nseg; ++k) v[i] += gld(partial, (row + k) * kStride + wave);
       }
-    };
-    if (nseg == 1)
-      add(std::integral_constant<int, 1>());
-    else
-      add(std::integral_constant<int, kSegs>());
+      schedule();
+      double acc = 0.0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) gsum[g][col + i] = acc[i];
-  }
-  __syncthreads();
-  if (wave == kTileWaves - 1 && lane == 0) {
-    // step-dependent scalars, computed once (powf is long) beside the other wavefronts' sums
-    const float t1 = (float)(c + 1);
-    sched[0] = schedule_lr(fo.opt, c);
-    sched[1] = 1.0f - powf(0.9f, t1);
-    sched[2] = 1.0f - powf(0.999f, t1);
-  }
-  for (int p = threadIdx.x; p < kStride; p += kTileThreads) {
-    double acc = 0.0;
+      for (int i = 0; i < kMaxTileBlocks / DIPS_WAVE; ++i) acc += lane + i * DIPS_WAVE < nblk ? (double)v[i] : 0.0;
+      acc = dips_wave_sum_d(acc);
+      if (lane == 0) gsh[wave] = (float)(acc * (double)fo.inv_b);
+    }
+    schedule();
+  } else {
+    const int col = min(4 * (wave % kRowWaves * DIPS_WAVE + lane), kStride - 4);
+    for (int g = wave / kRowWaves; g < kGroups && wave < kTeams * kRowWaves; g += kTeams) {
+      double acc[4] = {0.0, 0.0, 0.0, 0.0};
+      // 16 rows in flight: of 16 blocks, or of 4 blocks in kSegs parts each
+      auto add = [&](auto segs) {
+        constexpr int kS = decltype(segs)::value, kChunk = 16 / kS;
+        for (int b0 = g; b0 < nblk; b0 += kChunk * kGroups) {
+          row4 v[kChunk][kS];
 #pragma unroll
-    for (int g = 0; g < kGroups; ++g) acc += gsum[g][p];
-    gsh[p] = (float)(acc * (double)fo.inv_b);
+          for (int j = 0; j < kChunk; ++j)
+#pragma unroll
+            for (int k = 0; k < kS; ++k)
+              v[j][k] =
+                  *(global_row4*)(partial + ((int64_t)min(b0 + j * kGroups, nblk - 1) * kS + k) * kStride + col);
+          schedule();
+#pragma unroll
+          for (int j = 0; j < kChunk; ++j)
+            if (b0 + j * kGroups < nblk) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                float t = v[j][0][i];
+#pragma unroll
+                for (int k = 1; k < kS; ++k) t += v[j][k][i];
+                acc[i] += (double)t;
+              }
+            }
+        }
+      };
+      if (nseg == 1)
+        add(std::integral_constant<int, 1>());
+      else
+        add(std::integral_constant<int, kSegs>());
+#pragma unroll
+      for (int i = 0; i < 4; ++i) gsum[g][col + i] = acc[i];
+    }
+    schedule();
+    __syncthreads();
+    for (int p = threadIdx.x; p < kStride; p += kTileThreads) {
+      double acc = 0.0;
+#pragma unroll
+      for (int g = 0; g < kGroups; ++g) acc += gsum[g][p];
+      gsh[p] = (float)(acc * (double)fo.inv_b);
+    }
   }
   __syncthreads();
   double sq = 0.0;
