@@ -1422,12 +1422,22 @@ __global__ __launch_bounds__((kBT * bwd_groups<NBm, NBp, kStored>()), 2) void mf
     float xin_next = item_input(T, item_of(0), ee, kq);
     float seed_next = seed_of(item_of(0));
     // the stored activations of a round's tile (layers 1..L-1), loaded for round rd + 1 inside round rd
-    // once its activations are dead.  Past the phase's tiles the last one's are read again (finite, seeds zero).
+    // once its activations are dead.  Past the phase's tiles the split form, whose registers a conditional fill with
+    // zeros would spill, reads the last one's again (finite, seeds zero); the others, which it costs a wait in every round
+    // (2x12..16, 120 K tiles: 103 -> 109 us), load nothing.
     float act_n[L][4 * NB];
     auto load_round = [&](int64_t rd) {
       if constexpr (kStored) {
-        const int64_t tile = min((rd * nblk + bid) * kBW + wave, ntiles - 1);
-        load_act<L, NB>(act_in + ((plus ? tile : ntp + tile) * act_f4) * 64 + lane, act_n);
+        const int64_t tile = (rd * nblk + bid) * kBW + wave;
+        if (BP::kSplit || tile < ntiles) {
+          const int64_t at = BP::kSplit ? min(tile, ntiles - 1) : tile;
+          load_act<L, NB>(act_in + ((plus ? at : ntp + at) * act_f4) * 64 + lane, act_n);
+        } else {
+#pragma unroll
+          for (int l = 1; l < L; ++l)
+#pragma unroll
+            for (int q = 0; q < 4 * NB; ++q) act_n[l][q] = 0.0f;
+        }
       }
     };
     load_round(0);
@@ -1451,7 +1461,9 @@ __global__ __launch_bounds__((kBT * bwd_groups<NBm, NBp, kStored>()), 2) void mf
       } else {
         tile_forward<L, NB>(lds, xin, act);
       }
-      auto prefetch = [&] { load_round(rd + 1); };
+      auto prefetch = [&] {
+        if (BP::kSplit || rd + 1 < rounds) load_round(rd + 1);
+      };
       if constexpr (BP::kSplit)
         split_backward<L, NB>(lds, edges + 64 * NB, seed, xin, act, stage, G, prefetch);
       else
